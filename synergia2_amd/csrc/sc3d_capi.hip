@@ -660,7 +660,7 @@ int sc3d_set_post_kick_maps(sc3d_ctx* c, const sc3d_map_slice* slices, int nslic
             return fail(SC3D_ERR_ARG, "sc3d_set_post_kick_maps: unknown slice kind");
         if (slices[k].kind == SC3D_MAP_QUADRUPOLE && slices[k].yoshida_steps < 1)
             return fail(SC3D_ERR_ARG, "sc3d_set_post_kick_maps: yoshida_steps < 1");
-        c->post.s[k] = slices[k];
+        c->post.s[k] = prepare_slice(slices[k]);
     }
     c->post.n = nslices;
     return SC3D_OK;

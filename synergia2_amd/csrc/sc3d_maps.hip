@@ -9,56 +9,52 @@
 
 namespace sc3d {
 
-__global__ __launch_bounds__(kThreads) void k_maps(double* __restrict__ parts, int64_t stride,
-                                                   const uint8_t* __restrict__ masks, int64_t n,
-                                                   MapProgram prog)
+__device__ __forceinline__ void maps_pass(double* __restrict__ parts, int64_t stride,
+                                          const uint8_t* __restrict__ masks, int64_t n,
+                                          const MapProgram& prog)
 {
-    for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * kThreads) {
-        if (!masks[i]) continue;
-        double x = parts[i], xp = parts[i + stride], y = parts[i + 2 * stride],
-               yp = parts[i + 3 * stride], cdt = parts[i + 4 * stride];
-        const double dpop = parts[i + 5 * stride];
-        for (int k = 0; k < prog.n; ++k)
-            apply_slice(prog.s[k], x, xp, y, yp, cdt, dpop, prog.ref_p, prog.mass);
-        parts[i] = x;
-        parts[i + stride] = xp;
-        parts[i + 2 * stride] = y;
-        parts[i + 3 * stride] = yp;
-        parts[i + 4 * stride] = cdt;
-    }
+    const int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x;
+    if (i >= n || !masks[i]) return;
+    double x, xp, y, yp, cdt;
+    auto load = [&](int64_t j) {
+        x = parts[j];
+        xp = parts[j + stride];
+        y = parts[j + 2 * stride];
+        yp = parts[j + 3 * stride];
+        cdt = parts[j + 4 * stride];
+    };
+    load(i);
+    apply_program(prog, x, xp, y, yp, cdt, parts[i + 5 * stride],
+                  [&] { load(reread_index(i)); });
+    parts[i] = x;
+    parts[i + stride] = xp;
+    parts[i + 2 * stride] = y;
+    parts[i + 3 * stride] = yp;
+    parts[i + 4 * stride] = cdt;
+}
+
+__global__ __launch_bounds__(kThreads, 4) void k_maps(double* __restrict__ parts, int64_t stride,
+                                                      const uint8_t* __restrict__ masks,
+                                                      int64_t n, MapProgram prog)
+{
+    maps_pass(parts, stride, masks, n, prog);
 }
 
 // Served form: the scheduled program before the kick (first step only).
-__global__ __launch_bounds__(kThreads) void k_maps_sched(double* __restrict__ parts,
-                                                         int64_t stride,
-                                                         const uint8_t* __restrict__ masks,
-                                                         int64_t n, const MapProgram* progs,
-                                                         const StepCtl* ctl)
+__global__ __launch_bounds__(kThreads, 4) void k_maps_sched(double* __restrict__ parts,
+                                                            int64_t stride,
+                                                            const uint8_t* __restrict__ masks,
+                                                            int64_t n, const MapProgram* progs,
+                                                            const StepCtl* ctl)
 {
     if (ctl->done || ctl->first_prog < 0) return;
-    const MapProgram& prog = progs[ctl->first_prog];
-    for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * kThreads) {
-        if (!masks[i]) continue;
-        double x = parts[i], xp = parts[i + stride], y = parts[i + 2 * stride],
-               yp = parts[i + 3 * stride], cdt = parts[i + 4 * stride];
-        const double dpop = parts[i + 5 * stride];
-        for (int k = 0; k < prog.n; ++k)
-            apply_slice(prog.s[k], x, xp, y, yp, cdt, dpop, prog.ref_p, prog.mass);
-        parts[i] = x;
-        parts[i + stride] = xp;
-        parts[i + 2 * stride] = y;
-        parts[i + 3 * stride] = yp;
-        parts[i + 4 * stride] = cdt;
-    }
+    maps_pass(parts, stride, masks, n, progs[ctl->first_prog]);
 }
 
 void launch_maps_sched(double* parts, int64_t stride, const uint8_t* masks, int64_t n,
                        const Sched& sc, hipStream_t st)
 {
-    int64_t blocks = (n + kThreads - 1) / kThreads;
-    if (blocks > 8192) blocks = 8192;
+    const int64_t blocks = (n + kThreads - 1) / kThreads;
     if (blocks < 1) return;
     hipLaunchKernelGGL(k_maps_sched, dim3(unsigned(blocks)), dim3(kThreads), 0, st, parts, stride,
                        masks, n, sc.progs, sc.ctl);
@@ -76,7 +72,7 @@ double sc3d_reference_cdt(const sc3d_map_slice* s, double ref_p, double mass)
     double x = 0.0, xp = 0.0, y = 0.0, yp = 0.0, cdt = 0.0;
     sc3d_map_slice z = *s;
     z.ref_cdt = 0.0;
-    sc3d::apply_slice(z, x, xp, y, yp, cdt, 0.0, ref_p, mass);
+    sc3d::apply_slice(sc3d::prepare_slice(z), x, xp, y, yp, cdt, 0.0, ref_p, mass);
     return cdt;
 }
 
@@ -95,12 +91,11 @@ int sc3d_apply_maps(const sc3d_bunch* b, const sc3d_map_slice* slices, int nslic
     if (!b->parts || !b->masks || b->stride < n)
         return sc3d_internal_fail(SC3D_ERR_ARG, "sc3d_apply_maps: bad bunch");
     sc3d::MapProgram prog{};
-    for (int k = 0; k < nslices; ++k) prog.s[k] = slices[k];
+    for (int k = 0; k < nslices; ++k) prog.s[k] = sc3d::prepare_slice(slices[k]);
     prog.n = nslices;
     prog.ref_p = b->ref_p;
     prog.mass = b->mass;
-    int64_t blocks = (n + sc3d::kThreads - 1) / sc3d::kThreads;
-    if (blocks > 8192) blocks = 8192;
+    const int64_t blocks = (n + sc3d::kThreads - 1) / sc3d::kThreads;
     hipLaunchKernelGGL(sc3d::k_maps, dim3(unsigned(blocks)), dim3(sc3d::kThreads), 0,
                        static_cast<hipStream_t>(stream), b->parts, b->stride, b->masks, n, prog);
     if (hipGetLastError() != hipSuccess)

@@ -1413,9 +1413,10 @@ __global__ __launch_bounds__(kThreads) void k_efield(const R* __restrict__ phi, 
 // 0 <= idx < g-1 in all axes; trilinear Ez -> energy kick on dp/p, then Ey
 // -> y', then Ex -> x', each interpolation summed in the reference's corner
 // order.  Momenta accumulate in FP64 for every precision.
-// MAPS: the map program that follows the kick in the split-operator
-// sequence is applied to every active particle in the same pass (one read
-// and one write of the six coordinates for kick + maps).
+// k_kick also applies the map program that follows the kick in the
+// split-operator sequence to every active particle in the same pass (one read
+// and one write of the six coordinates for kick + maps); SCHED: the served
+// form's scheduled program instead of the one passed by value.
 // COPY (the apply that reordered the bunch): the particles are read from the
 // cell-sorted copy the reorder gathered (src: 7 columns of stride n, and its
 // masks), and every particle's 7 columns and mask are written to the bunch
@@ -1431,8 +1432,8 @@ __device__ __forceinline__ double kick_factor(const DomainRec& d)
     return d.factor * d.w0 * (peak > 0.0f ? double(peak) : 1.0);
 }
 
-template <typename R, bool MAPS, bool COPY>
-__global__ __launch_bounds__(kThreads) void k_kick(double* __restrict__ parts, int64_t stride,
+template <typename R, bool COPY, bool SCHED>
+__global__ __launch_bounds__(kThreads, 4) void k_kick(double* __restrict__ parts, int64_t stride,
                                                    uint8_t* __restrict__ masks, int64_t n,
                                                    int gx, int gy, int gz,
                                                    const DomainRec* __restrict__ dom,
@@ -1442,73 +1443,73 @@ __global__ __launch_bounds__(kThreads) void k_kick(double* __restrict__ parts, i
                                                    const uint8_t* __restrict__ smasks)
 {
     if (dom->error) return;
-    // served form: the program fused after the kick comes from the schedule
-    const MapProgram* __restrict__ sp = (MAPS && sc.progs) ? sc.progs + sc.ctl->after_prog
-                                                            : nullptr;
+    const MapProgram* __restrict__ sp = SCHED ? sc.progs + sc.ctl->after_prog : nullptr;
     const double lx = dom->left[0], ly = dom->left[1], lz = dom->left[2];
     const double ihx = dom->inv_h[0], ihy = dom->inv_h[1], ihz = dom->inv_h[2];
     const double factor = kick_factor<R>(*dom);
     const double* __restrict__ rd = COPY ? src : parts;
     const int64_t rs = COPY ? n : stride;
-    for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * kThreads) {
-        const uint8_t on = COPY ? smasks[i] : masks[i];
-        if (!COPY && !on) continue;
-        // all six coordinates are loaded up front (independent loads in flight)
-        double x = rd[i], y = rd[i + 2 * rs], cdt = rd[i + 4 * rs];
-        double xp = rd[i + rs], yp = rd[i + 3 * rs], dpop = rd[i + 5 * rs];
-        double ox, oy, oz;
-        const int ix = cell_index(x, lx, ihx, ox);
-        const int iy = cell_index(y, ly, ihy, oy);
-        const int iz = cell_index(cdt, lz, ihz, oz);
-        const bool in = on && (ix >= 0 && ix < gx - 1) && (iy >= 0 && iy < gy - 1) &&
-                        (iz >= 0 && iz < gz - 1);
-        if (COPY) {
-            masks[i] = on;
-            parts[i + 6 * stride] = rd[i + 6 * rs];
-        }
-        if (!MAPS && !COPY && !in) continue;
-        if (in) {
-            const double aox = 1.0 - ox, aoy = 1.0 - oy, aoz = 1.0 - oz;
-            const int64_t b0 = (int64_t(iz) * gy + iy) * gx + ix;
-            const int64_t b1 = b0 + int64_t(gx) * gy;
-            typename vec4<R>::type e[8] = {E[b0],  E[b0 + 1],  E[b0 + gx],  E[b0 + gx + 1],
-                                           E[b1],  E[b1 + 1],  E[b1 + gx],  E[b1 + gx + 1]};
-            const double w[8] = {aoz * aoy * aox, aoz * aoy * ox, aoz * oy * aox, aoz * oy * ox,
-                                 oz * aoy * aox,  oz * aoy * ox,  oz * oy * aox,  oz * oy * ox};
-            double vz = w[0] * double(e[0].z), vy = w[0] * double(e[0].y),
-                   vx = w[0] * double(e[0].x);
-#pragma unroll
-            for (int c = 1; c < 8; ++c) {
-                vz += w[c] * double(e[c].z);
-                vy += w[c] * double(e[c].y);
-                vx += w[c] * double(e[c].x);
-            }
-            const double p = pref + dpop * pref;
-            const double Eoc_i = sqrt(p * p + m * m);
-            const double Eoc_f = Eoc_i + factor * (-pref) * vz;
-            dpop += (sqrt(Eoc_f * Eoc_f - m * m) - sqrt(Eoc_i * Eoc_i - m * m)) / pref;
-            yp += factor * vy;
-            xp += factor * vx;
-        }
-        if (MAPS && on) {
-            if (sp) {
-                for (int k = 0; k < sp->n; ++k)
-                    apply_slice(sp->s[k], x, xp, y, yp, cdt, dpop, sp->ref_p, sp->mass);
-            } else {
-                for (int k = 0; k < prog.n; ++k)
-                    apply_slice(prog.s[k], x, xp, y, yp, cdt, dpop, prog.ref_p, prog.mass);
-            }
-        }
-        if (MAPS || COPY) {
-            parts[i] = x;
-            parts[i + 2 * stride] = y;
-            parts[i + 4 * stride] = cdt;
-        }
-        parts[i + stride] = xp;
-        parts[i + 3 * stride] = yp;
-        parts[i + 5 * stride] = dpop;
+    const int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x;
+    if (i >= n) return;
+    const uint8_t on = COPY ? smasks[i] : masks[i];
+    if (!COPY && !on) return;
+    // all six coordinates are loaded up front (independent loads in flight)
+    double x = rd[i], y = rd[i + 2 * rs], cdt = rd[i + 4 * rs];
+    double xp = rd[i + rs], yp = rd[i + 3 * rs], dpop = rd[i + 5 * rs];
+    double ox, oy, oz;
+    const int ix = cell_index(x, lx, ihx, ox);
+    const int iy = cell_index(y, ly, ihy, oy);
+    const int iz = cell_index(cdt, lz, ihz, oz);
+    const bool in = on && (ix >= 0 && ix < gx - 1) && (iy >= 0 && iy < gy - 1) &&
+                    (iz >= 0 && iz < gz - 1);
+    if (COPY) {
+        masks[i] = on;
+        parts[i + 6 * stride] = rd[i + 6 * rs];
     }
+    if (in) {
+        const double aox = 1.0 - ox, aoy = 1.0 - oy, aoz = 1.0 - oz;
+        const int64_t b0 = (int64_t(iz) * gy + iy) * gx + ix;
+        const int64_t b1 = b0 + int64_t(gx) * gy;
+        typename vec4<R>::type e[8] = {E[b0],  E[b0 + 1],  E[b0 + gx],  E[b0 + gx + 1],
+                                       E[b1],  E[b1 + 1],  E[b1 + gx],  E[b1 + gx + 1]};
+        const double w[8] = {aoz * aoy * aox, aoz * aoy * ox, aoz * oy * aox, aoz * oy * ox,
+                             oz * aoy * aox,  oz * aoy * ox,  oz * oy * aox,  oz * oy * ox};
+        double vz = w[0] * double(e[0].z), vy = w[0] * double(e[0].y),
+               vx = w[0] * double(e[0].x);
+#pragma unroll
+        for (int c = 1; c < 8; ++c) {
+            vz += w[c] * double(e[c].z);
+            vy += w[c] * double(e[c].y);
+            vx += w[c] * double(e[c].x);
+        }
+        const double p = pref + dpop * pref;
+        const double Eoc_i = sqrt(p * p + m * m);
+        const double Eoc_f = Eoc_i + factor * (-pref) * vz;
+        dpop += (sqrt(Eoc_f * Eoc_f - m * m) - sqrt(Eoc_i * Eoc_i - m * m)) / pref;
+        yp += factor * vy;
+        xp += factor * vx;
+    }
+    if (on) {
+        const double xp0 = xp, yp0 = yp;
+        auto again = [&] {
+            const int64_t j = reread_index(i);
+            x = rd[j];
+            y = rd[j + 2 * rs];
+            cdt = rd[j + 4 * rs];
+            xp = xp0;
+            yp = yp0;
+        };
+        if (SCHED)
+            apply_program(*sp, x, xp, y, yp, cdt, dpop, again);
+        else
+            apply_program(prog, x, xp, y, yp, cdt, dpop, again);
+    }
+    parts[i] = x;
+    parts[i + 2 * stride] = y;
+    parts[i + 4 * stride] = cdt;
+    parts[i + stride] = xp;
+    parts[i + 3 * stride] = yp;
+    parts[i + 5 * stride] = dpop;
 }
 
 // The kick without maps over windows of the bunch storage (kKickPer
@@ -1523,7 +1524,7 @@ __global__ __launch_bounds__(kThreads) void k_kick(double* __restrict__ parts, i
 // copies of the field values.  Measured (kick us, 4e6 FP64 on 64x64x128 /
 // 1.6e7 FP32 on 128x128x256, one run): k_kick 75.7 / 242; 2 particles per
 // lane and 1024 nodes 69.4 / 224; 4 and 2048 nodes 70.5 / 240; 1 and 512
-// nodes 73.9 / 234.  With the maps fused (k_kick<R, true>) the extra
+// nodes 73.9 / 234.  With the maps fused (k_kick) the extra
 // registers of the tile version cost more than the gathers save: the fused
 // kick stays on k_kick.
 constexpr int kKickPer = 2;
@@ -2048,16 +2049,15 @@ void launch_kick(double* parts, int64_t stride, uint8_t* masks, int64_t n, int g
                                stride, masks, n, gx, gy, gz, dom, E, pref, m, src, smasks);
         return;
     }
-    // kick + maps: up to 32768 blocks (measured at 1.6e7 particles: 240 us,
-    // against 251 with 8192 blocks, 272 with 4096 and 247 with one particle
-    // per thread, for the kick alone)
-    const dim3 grid(grid_for(n, 32768));
-    if (copy)
-        hipLaunchKernelGGL((k_kick<R, true, true>), grid, dim3(kThreads), 0, st, parts, stride,
-                           masks, n, gx, gy, gz, dom, E, pref, m, prog, sc, src, smasks);
+    const dim3 grid(unsigned((n + kThreads - 1) / kThreads));
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, parts, stride, masks, n, gx, gy,
+                           gz, dom, E, pref, m, prog, sc, src, smasks);
+    };
+    if (sc.progs)
+        copy ? launch(k_kick<R, true, true>) : launch(k_kick<R, false, true>);
     else
-        hipLaunchKernelGGL((k_kick<R, true, false>), grid, dim3(kThreads), 0, st, parts, stride,
-                           masks, n, gx, gy, gz, dom, E, pref, m, prog, sc, src, smasks);
+        copy ? launch(k_kick<R, true, false>) : launch(k_kick<R, false, false>);
 }
 
 void launch_populate(double* parts, int64_t stride, int64_t n, uint8_t* masks,

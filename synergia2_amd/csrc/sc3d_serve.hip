@@ -442,7 +442,7 @@ int sc3d_server_submit(sc3d_server* s, const sc3d_job_spec* spec, int64_t* id)
         for (int k = 0; k < T; ++k) {
             MapProgram& p = j->progs[size_t(t) * T + k];
             p = MapProgram{};
-            for (int q = 0; q < tab[k].n; ++q) p.s[q] = tab[k].s[q];
+            for (int q = 0; q < tab[k].n; ++q) p.s[q] = prepare_slice(tab[k].s[q]);
             p.n = tab[k].n;
             p.ref_p = spec->ref_p;
             p.mass = spec->mass;
