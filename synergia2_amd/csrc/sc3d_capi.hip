@@ -770,7 +770,7 @@ int sc3d_tail_fraction(sc3d_ctx* c, const sc3d_bunch* b, const double center[6],
         return fail(SC3D_ERR_ARG, "sc3d_tail_fraction: bad bunch");
     HIP_TRY(hipSetDevice(c->device));
     if (!c->tails)
-        if (int rc = dmalloc(c, &c->tails, 8)) return rc;
+        if (int rc = dmalloc(c, &c->tails, kTailWords)) return rc;
     TailArgs a{};
     for (int j = 0; j < 6; ++j) {
         a.c[j] = center[j];

@@ -92,6 +92,9 @@ struct TailArgs {
     double c[6];    // centre per plane
     double lim[6];  // |p - c| beyond this counts as tail
 };
+constexpr int kTailBlocks = 1024;
+// counts: kTailWords words, the six counts first, the blocks' counts behind
+constexpr int kTailWords = 8 + 6 * kTailBlocks / 2;
 void launch_tail_counts(const double* parts, int64_t stride, const uint8_t* masks, int64_t n,
                         const TailArgs& a, unsigned long long* counts, hipStream_t st);
 void launch_populate(double* parts, int64_t stride, int64_t n, uint8_t* masks,
