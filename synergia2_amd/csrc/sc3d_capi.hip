@@ -111,7 +111,7 @@ Geometry geometry_of(const sc3d_options& o, bool all_generic = false)
         g.plan[a] = AnyPlan{};
         g.tw_any[a] = -1;
         if (!g.tuned[a]) {
-            g.plan[a] = any_plan(len[a]);
+            g.plan[a] = any_plan(len[a], o.precision == SC3D_PRECISION_FP32_GRID);
             g.tw_any[a] = off;
             off += len[a];
         }

@@ -27,6 +27,7 @@
 // passes and stored as that octant only.
 #include <type_traits>
 
+#include "sc3d_dft.h"
 #include "sc3d_green.h"
 #include "sc3d_internal.h"
 
@@ -102,114 +103,6 @@ using RowLines = CappedLines<M, K, T2, HalfLines<M>::value>;
 // the Green's function column passes (two real columns per line)
 template <int L, typename T2>
 using GreenLines = CappedLines<L, 1, T2, HalfLines<L>::value>;
-
-// a * w^m, w = e^(-2 pi i / 16) (inverse: e^(+2 pi i / 16)), written with
-// the cosine c and sine s of 2 pi m / 16 (fused multiply-adds: the build
-// contracts nothing by itself)
-template <bool INV, typename T2, typename F>
-__device__ __forceinline__ T2 rot16(T2 a, F c, F s)
-{
-    T2 o;
-    if (!INV) { o.x = fma(a.x, c, a.y * s); o.y = fma(a.y, c, -(a.x * s)); }
-    else      { o.x = fma(a.x, c, -(a.y * s)); o.y = fma(a.y, c, a.x * s); }
-    return o;
-}
-
-// a * w for a twiddle w (INV: a * conj(w)), fused multiply-adds
-template <bool INV, typename T2>
-__device__ __forceinline__ T2 twmul(T2 a, T2 w)
-{
-    T2 o;
-    if (!INV) { o.x = fma(a.x, w.x, -(a.y * w.y)); o.y = fma(a.x, w.y, a.y * w.x); }
-    else      { o.x = fma(a.x, w.x, a.y * w.y);    o.y = fma(a.y, w.x, -(a.x * w.y)); }
-    return o;
-}
-
-template <int R, bool INV, typename T2>
-__device__ __forceinline__ void dft_small(T2* v)
-{
-    if constexpr (R == 16) {
-        // 16 = 4 x 4: inputs x[4 n1 + n2]; a length-4 DFT over n1 for each
-        // n2 gives A[n2][k1], then A[n2][k1] w^(n2 k1), then a length-4 DFT
-        // over n2 for each k1 gives X[k1 + 4 k2]
-        using F = decltype(v[0].x);
-        const F c1 = F(0.92387953251128675613), s1 = F(0.38268343236508977173);
-        const F c2 = F(0.70710678118654752440);
-        T2 a[4][4];
-#pragma unroll
-        for (int n2 = 0; n2 < 4; ++n2) {
-#pragma unroll
-            for (int n1 = 0; n1 < 4; ++n1) a[n2][n1] = v[4 * n1 + n2];
-            dft_small<4, INV>(a[n2]);
-        }
-        a[1][1] = rot16<INV>(a[1][1], c1, s1);   // w^1
-        a[1][2] = rot16<INV>(a[1][2], c2, c2);   // w^2
-        a[1][3] = rot16<INV>(a[1][3], s1, c1);   // w^3
-        a[2][1] = rot16<INV>(a[2][1], c2, c2);   // w^2
-        {                                        // w^4 = -i (inverse: +i)
-            T2 t = a[2][2];
-            if (!INV) { a[2][2].x = t.y;  a[2][2].y = -t.x; }
-            else      { a[2][2].x = -t.y; a[2][2].y = t.x; }
-        }
-        a[2][3] = rot16<INV>(a[2][3], -c2, c2);  // w^6
-        a[3][1] = rot16<INV>(a[3][1], s1, c1);   // w^3
-        a[3][2] = rot16<INV>(a[3][2], -c2, c2);  // w^6
-        a[3][3] = rot16<INV>(a[3][3], -c1, -s1); // w^9
-#pragma unroll
-        for (int k1 = 0; k1 < 4; ++k1) {
-            T2 b[4] = {a[0][k1], a[1][k1], a[2][k1], a[3][k1]};
-            dft_small<4, INV>(b);
-#pragma unroll
-            for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = b[k2];
-        }
-    } else if constexpr (R == 8) {
-        // y_k = E_(k mod 4) + w8^k O_(k mod 4), E/O = DFT4 of the even/odd
-        // inputs, w8 = e^(-i pi/4) (inverse: conjugate), w8^(k+4) = -w8^k
-        T2 e[4] = {v[0], v[2], v[4], v[6]};
-        T2 o[4] = {v[1], v[3], v[5], v[7]};
-        dft_small<4, INV>(e);
-        dft_small<4, INV>(o);
-        using F = decltype(v[0].x);
-        const F c = F(0.70710678118654752440);
-        T2 t1, t2, t3;
-        if (!INV) {
-            t1.x = (o[1].x + o[1].y) * c; t1.y = (o[1].y - o[1].x) * c;  // (1 - i) c
-            t2.x = o[2].y;                t2.y = -o[2].x;                // -i
-            t3.x = (o[3].y - o[3].x) * c; t3.y = -(o[3].x + o[3].y) * c; // (-1 - i) c
-        } else {
-            t1.x = (o[1].x - o[1].y) * c; t1.y = (o[1].x + o[1].y) * c;  // (1 + i) c
-            t2.x = -o[2].y;               t2.y = o[2].x;                 // i
-            t3.x = -(o[3].x + o[3].y) * c; t3.y = (o[3].x - o[3].y) * c; // (-1 + i) c
-        }
-        v[0].x = e[0].x + o[0].x; v[0].y = e[0].y + o[0].y;
-        v[4].x = e[0].x - o[0].x; v[4].y = e[0].y - o[0].y;
-        v[1].x = e[1].x + t1.x;   v[1].y = e[1].y + t1.y;
-        v[5].x = e[1].x - t1.x;   v[5].y = e[1].y - t1.y;
-        v[2].x = e[2].x + t2.x;   v[2].y = e[2].y + t2.y;
-        v[6].x = e[2].x - t2.x;   v[6].y = e[2].y - t2.y;
-        v[3].x = e[3].x + t3.x;   v[3].y = e[3].y + t3.y;
-        v[7].x = e[3].x - t3.x;   v[7].y = e[3].y - t3.y;
-    } else if constexpr (R == 2) {
-        T2 a = v[0], b = v[1];
-        v[0].x = a.x + b.x; v[0].y = a.y + b.y;
-        v[1].x = a.x - b.x; v[1].y = a.y - b.y;
-    } else {
-        T2 a, b, c, d;
-        a.x = v[0].x + v[2].x; a.y = v[0].y + v[2].y;
-        b.x = v[0].x - v[2].x; b.y = v[0].y - v[2].y;
-        c.x = v[1].x + v[3].x; c.y = v[1].y + v[3].y;
-        d.x = v[1].x - v[3].x; d.y = v[1].y - v[3].y;
-        v[0].x = a.x + c.x; v[0].y = a.y + c.y;
-        v[2].x = a.x - c.x; v[2].y = a.y - c.y;
-        if (!INV) {  // y1 = b - i d, y3 = b + i d
-            v[1].x = b.x + d.y; v[1].y = b.y - d.x;
-            v[3].x = b.x - d.y; v[3].y = b.y + d.x;
-        } else {     // y1 = b + i d, y3 = b - i d
-            v[1].x = b.x - d.y; v[1].y = b.y + d.x;
-            v[3].x = b.x + d.y; v[3].y = b.y - d.x;
-        }
-    }
-}
 
 // One Stockham autosort pass of radix R on NL lines of length L in LDS
 // (Govindaraju et al., SC'08 formulation): butterfly j reads j + r*L/R,

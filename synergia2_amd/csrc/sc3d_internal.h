@@ -11,15 +11,18 @@ namespace sc3d {
 // doubled complex grid (Dy rows of Hx each); Ghat holds the real Green's
 // spectrum for kz <= gz, ky <= gy, kx <= gx.
 // Radix plan of a transform of any length L <= kAnyMaxLen for the generic
-// passes (sc3d_fft_any.hip): factors 4, then primes ascending.
+// passes (sc3d_fft_any.hip).
 constexpr int kAnyMaxLen = 1024;
-constexpr int kAnyMaxPasses = 16;
+constexpr int kAnyMaxPasses = 10;
 struct AnyPlan {
     int L;
     int np;
+    int tpl;  // threads of a line that take every register pass in one round
     int R[kAnyMaxPasses];
+    uint32_t ns_magic[kAnyMaxPasses];    // ceil(2^32 / product of the earlier radices)
+    uint32_t back_magic[kAnyMaxPasses];  // ... of the later ones (radices in reverse)
 };
-AnyPlan any_plan(int L);
+AnyPlan any_plan(int L, bool fp32);
 
 struct Geometry {
     int gx, gy, gz;
