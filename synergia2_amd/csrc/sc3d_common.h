@@ -52,6 +52,27 @@ __device__ __forceinline__ int cell_index(double pos, double left, double inv_h,
     return idx;
 }
 
+// The cell of a position that the deposit and the kick touch: index in
+// [0, g-2].  Same index and offset as cell_index there (for s >= 0 truncation
+// is floor, and floor(s) <= g-2 exactly when s < g-1); otherwise false and
+// both unspecified.
+__device__ __forceinline__ bool grid_cell(double pos, double left, double inv_h, int g, int& idx,
+                                          double& off)
+{
+    const double s = (pos - left) * inv_h - 0.5;
+    const bool in = s >= 0.0 && s < double(g - 1);
+    idx = static_cast<int>(in ? s : 0.0);
+    off = s - idx;
+    return in;
+}
+
+// n / d for n * d < 2^32, d >= 2, as umulhi(n, magic).
+__device__ __forceinline__ uint32_t small_magic(uint32_t d) { return 0xffffffffu / d + 1u; }
+__device__ __forceinline__ int small_div(int n, uint32_t magic)
+{
+    return int(__umulhi(uint32_t(n), magic));
+}
+
 // Device-side control of the applies of one context in the served form
 // (kernels take it as a nullable pointer; null = the host decides, as in
 // sc3d_apply).  k_step_begin opens each apply: which scheduled map programs

@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/sc3d_capi.h"
+#include "sc3d_exact.h"
 
 namespace sc3d {
 
@@ -137,8 +138,7 @@ struct MapProgram {
 // three (46 instructions), and the results are the same bits:
 //   y  ~ 1/sqrt(a), a = dp^2 - x'^2 - y'^2: hardware seed, one third-order
 //      step, about 1 ulp;
-//   s  = sqrt(a) = g + (a - g^2) y/2 with g = a y: Newton's residual form with
-//      one rounding (P. Markstein, IBM J. Res. Dev. 34, 1990);
+//   s  = sqrt(a) from y (sc3d_exact.h);
 //   1/s = y + y (1 - s y), exact residual, the same reference; it can miss
 //      when s has an all-ones significand, which `ones` records;
 //   the path length sqrt(D2/beta^2) equals |l| C / s, C = dp/beta, up to a few
@@ -197,11 +197,8 @@ __device__ __forceinline__ void fast_drift(FastDrift& f, double& x, double xp, d
 {
     const double a = f.dp2 - xp * xp - yp * yp;
     f.a_low = min(f.a_low, int32_t(__double_as_longlong(a) >> 32));
-    const double y0 = __builtin_amdgcn_rsq(a);
-    const double e = __builtin_fma(-(a * y0), y0, 1.0);
-    const double yr = __builtin_fma(y0 * e, __builtin_fma(e, 0.375, 0.5), y0);
-    const double g = a * yr;
-    const double s = __builtin_fma(__builtin_fma(-g, g, a), 0.5 * yr, g);
+    const double yr = rsqrt_near(a);
+    const double s = sqrt_from(a, yr);
     f.ones = max(f.ones, uint32_t(__double_as_longlong(s)));
     const double inv_npz = __builtin_fma(yr, __builtin_fma(-s, yr, 1.0), yr);
     const double lxpr = xp * l * inv_npz;
