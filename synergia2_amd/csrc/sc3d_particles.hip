@@ -1132,6 +1132,11 @@ __global__ __launch_bounds__(kThreads) void k_deposit(const double* __restrict__
 // eighth / sixteenth / thirty-second rotated first, or none, 54.6-54.8 /
 // 55.4-55.5 / 54.3-54.5 / 56.1-56.3 at 4e6 and 200.6-200.7 / 201.3-202.4 /
 // 201.8-202.3 / 203.5 at 1.6e7; 3 slots per thread 57.4-57.6 / 212.2-212.5.
+// Weights formed in the lane's corner order, offsets once per thread and the
+// flush's divisions by multiplication (248 -> 176 VALU instructions per
+// particle): 46.9 -> 42.3 us per launch at 4e6 FP64, 226 -> 218 at 1.6e7 FP32
+// (about four runs a thread late in the sort period; then the LDS atomics and
+// the four blocks a CU holds are the limit).
 constexpr int kTileThreads = 256;
 constexpr int kTilePer = 4;                             // consecutive slots per thread
 constexpr int kTileWindow = kTileThreads * kTilePer;    // slots per block
@@ -1165,78 +1170,73 @@ __device__ __forceinline__ int wave_max(int v)
                max(__builtin_amdgcn_readlane(v, 47), __builtin_amdgcn_readlane(v, 63)));
 }
 
-// Corner weights of one particle in the reference's order, w0*wx*wy*wz left
-// to right (deposit.cc:366-391); corner c = (x bit 0, y bit 1, z bit 2).
-__device__ __forceinline__ void tile_weights(double w0, double ox, double oy, double oz,
-                                             double (&w)[8])
-{
-    const double aox = 1.0 - ox, aoy = 1.0 - oy, aoz = 1.0 - oz;
+// Corners in this lane's order: position k is corner k ^ (lane mod 8) (x bit
+// 0, y bit 1, z bit 2), so that the lanes of one cell add to eight different
+// nodes at a time.  The order enters where the three factor pairs are formed,
+// so weights and run sums come out in it and nothing is permuted afterwards
+// (permuting the sums by register swaps at every run took 48 instructions).
+struct LaneCorners {
+    bool sx, sy, sz;
+    __device__ __forceinline__ explicit LaneCorners(int lane)
+        : sx(lane & 1), sy(lane & 2), sz(lane & 4) {}
+    // weights in the reference's order of products, w0*wx*wy*wz left to right
+    // (deposit.cc:366-391)
+    __device__ __forceinline__ void weights(double w0, double ox, double oy, double oz,
+                                            double (&w)[8]) const
+    {
+        const double aox = 1.0 - ox, aoy = 1.0 - oy, aoz = 1.0 - oz;
+        const double fx[2] = {sx ? ox : aox, sx ? aox : ox};
+        const double fy[2] = {sy ? oy : aoy, sy ? aoy : oy};
+        const double fz[2] = {sz ? oz : aoz, sz ? aoz : oz};
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const double wx = (c & 1) ? ox : aox, wy = (c & 2) ? oy : aoy, wz = (c & 4) ? oz : aoz;
-        w[c] = w0 * wx * wy * wz;
+        for (int k = 0; k < 8; ++k) w[k] = w0 * fx[k & 1] * fy[(k >> 1) & 1] * fz[k >> 2];
     }
-}
-
-// Adds the eight corner sums of the cell at tile offset b0 (box of nx x ny
-// x .. nodes): at step k corner k ^ (lane mod 8), so the lanes of one cell
-// hit eight different nodes at a time.  The sums are permuted by three
-// conditional register swaps (an indexed pick would go through scratch).
-__device__ __forceinline__ void tile_add(double* tile, int b0, int nx, int ny, int lane,
-                                         const double (&w)[8])
-{
-    double v[8];
+    // node offsets in a box of nx x ny x .. nodes
+    __device__ __forceinline__ void offsets(int nx, int ny, int (&off)[8]) const
+    {
+        const int px[2] = {sx ? 1 : 0, sx ? 0 : 1};
+        const int py[2] = {sy ? nx : 0, sy ? 0 : nx};
+        const int pz[2] = {sz ? nx * ny : 0, sz ? 0 : nx * ny};
 #pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = w[c];
-    const int r = lane & 7;
-#pragma unroll
-    for (int bit = 1; bit < 8; bit <<= 1) {
-        const bool sw = r & bit;
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-            if (!(c & bit)) {
-                const double a = v[c], b = v[c | bit];
-                v[c] = sw ? b : a;
-                v[c | bit] = sw ? a : b;
-            }
+        for (int k = 0; k < 8; ++k) off[k] = px[k & 1] + py[(k >> 1) & 1] + pz[k >> 2];
     }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int c = k ^ r;  // v[k] holds corner c
-        const int off = ((c >> 2) * ny + ((c >> 1) & 1)) * nx + (c & 1);
-        unsafeAtomicAdd(&tile[b0 + off], v[k]);
-    }
-}
+};
 
 // This thread's particles into a tile whose box starts at (bx, by, bz):
 // consecutive particles of one cell summed first.
+template <int PER>
 __device__ __forceinline__ void tile_deposit(double* tile, int bx, int by, int bz, int nx, int ny,
-                                             int lane, double w0, const int (&ix)[kTilePer],
-                                             const int (&iy)[kTilePer], const int (&iz)[kTilePer],
-                                             const bool (&ok)[kTilePer],
-                                             const double (&ox)[kTilePer],
-                                             const double (&oy)[kTilePer],
-                                             const double (&oz)[kTilePer])
+                                             const LaneCorners& lc, double w0,
+                                             const int (&ix)[PER], const int (&iy)[PER],
+                                             const int (&iz)[PER], const bool (&ok)[PER],
+                                             const double (&ox)[PER], const double (&oy)[PER],
+                                             const double (&oz)[PER])
 {
+    int off[8];
+    lc.offsets(nx, ny, off);
     double s[8];
     int cur = -1;
+    auto add = [&] {
 #pragma unroll
-    for (int q = 0; q < kTilePer; ++q) {
+        for (int k = 0; k < 8; ++k) unsafeAtomicAdd(&tile[cur + off[k]], s[k]);
+    };
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
         if (!ok[q]) continue;
         const int b0 = ((iz[q] - bz) * ny + (iy[q] - by)) * nx + (ix[q] - bx);
         double w[8];
-        tile_weights(w0, ox[q], oy[q], oz[q], w);
+        lc.weights(w0, ox[q], oy[q], oz[q], w);
         if (b0 == cur) {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) s[c] += w[c];
+            for (int k = 0; k < 8; ++k) s[k] += w[k];
         } else {
-            if (cur >= 0) tile_add(tile, cur, nx, ny, lane, s);
+            if (cur >= 0) add();
 #pragma unroll
-            for (int c = 0; c < 8; ++c) s[c] = w[c];
+            for (int k = 0; k < 8; ++k) s[k] = w[k];
             cur = b0;
         }
     }
-    if (cur >= 0) tile_add(tile, cur, nx, ny, lane, s);
+    if (cur >= 0) add();
 }
 
 // The non-zero interior nodes of a tile (box at (bx, by, bz), nx x ny x ..,
@@ -1246,11 +1246,12 @@ __device__ __forceinline__ void tile_flush(const double* tile, int nodes, int fi
                                            int bx, int by, int bz, int nx, int ny, int gx, int gy,
                                            int gz, R* __restrict__ rho)
 {
+    const uint32_t mx = small_magic(nx), my = small_magic(ny);
     for (int e = first; e < nodes; e += step) {
         const double v = tile[e];
         if (v == 0.0) continue;
-        const int cx = bx + e % nx, r = e / nx;
-        const int cy = by + r % ny, cz = bz + r / ny;
+        const int r = small_div(e, mx), rz = small_div(r, my);
+        const int cx = bx + e - r * nx, cy = by + r - rz * ny, cz = bz + rz;
         if (cx > 0 && cx < gx - 1 && cy > 0 && cy < gy - 1 && cz > 0 && cz < gz - 1)
             unsafeAtomicAdd(rho + (int64_t(cz) * gy + cy) * gx + cx, R(v));
     }
@@ -1265,6 +1266,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     __shared__ int box[kTileWaves][6];
     if (dom->error) return;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const LaneCorners lc(lane);
     const double lx = dom->left[0], ly = dom->left[1], lz = dom->left[2];
     const double ihx = dom->inv_h[0], ihy = dom->inv_h[1], ihz = dom->inv_h[2];
     // precision form: unit weights (w0 and the unit-peak scale return at the kick)
@@ -1288,12 +1290,10 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
             y = parts[j + 2 * stride];
             z = parts[j + 4 * stride];
         }
-        ix[q] = cell_index(x, lx, ihx, ox[q]);
-        iy[q] = cell_index(y, ly, ihy, oy[q]);
-        iz[q] = cell_index(z, lz, ihz, oz[q]);
         // a particle outside [0, g-2] in any axis has no interior corner
-        ok[q] = m && ix[q] >= 0 && ix[q] <= gx - 2 && iy[q] >= 0 && iy[q] <= gy - 2 &&
-                iz[q] >= 0 && iz[q] <= gz - 2;
+        ok[q] = grid_cell(x, lx, ihx, gx, ix[q], ox[q]);
+        ok[q] = grid_cell(y, ly, ihy, gy, iy[q], oy[q]) && ok[q];
+        ok[q] = grid_cell(z, lz, ihz, gz, iz[q], oz[q]) && ok[q] && m;
         if (ok[q]) {
             lo[0] = min(lo[0], ix[q]); hi[0] = max(hi[0], ix[q]);
             lo[1] = min(lo[1], iy[q]); hi[1] = max(hi[1], iy[q]);
@@ -1330,7 +1330,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     if (nodes <= kTileNodes) {  // block-uniform
         for (int e = t; e < nodes; e += kTileThreads) tile[e] = 0.0;
         __syncthreads();
-        tile_deposit(tile, blo[0], blo[1], blo[2], nx, ny, lane, w0, ix, iy, iz, ok, ox, oy, oz);
+        tile_deposit(tile, blo[0], blo[1], blo[2], nx, ny, lc, w0, ix, iy, iz, ok, ox, oy, oz);
         __syncthreads();
         tile_flush<R>(tile, nodes, t, kTileThreads, blo[0], blo[1], blo[2], nx, ny, gx, gy, gz,
                       rho);
@@ -1345,7 +1345,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
         for (int e = lane; e < wn; e += 64) wtile[e] = 0.0;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        tile_deposit(wtile, lo[0], lo[1], lo[2], wnx, wny, lane, w0, ix, iy, iz, ok, ox, oy, oz);
+        tile_deposit(wtile, lo[0], lo[1], lo[2], wnx, wny, lc, w0, ix, iy, iz, ok, ox, oy, oz);
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
         tile_flush<R>(wtile, wn, lane, 64, lo[0], lo[1], lo[2], wnx, wny, gx, gy, gz, rho);
@@ -1368,9 +1368,10 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     for (int q = 0; q < kTilePer; ++q) {
         if (!ok[q]) continue;
         double w[8];
-        tile_weights(w0, ox[q], oy[q], oz[q], w);
+        lc.weights(w0, ox[q], oy[q], oz[q], w);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
+        for (int k = 0; k < 8; ++k) {
+            const int c = k ^ (lane & 7);
             const int cx = ix[q] + (c & 1), cy = iy[q] + ((c >> 1) & 1), cz = iz[q] + (c >> 2);
             if (!(cx > 0 && cx < gx - 1 && cy > 0 && cy < gy - 1 && cz > 0 && cz < gz - 1))
                 continue;
@@ -1378,9 +1379,9 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
             const int slot = int((uint32_t(node) * 2654435761u) >> 23) & (kCacheSlots - 1);
             const int held = atomicCAS(&ckey[slot], -1, node);
             if (held == -1 || held == node)
-                unsafeAtomicAdd(&cval[slot], w[c]);
+                unsafeAtomicAdd(&cval[slot], w[k]);
             else
-                unsafeAtomicAdd(rho + node, R(w[c]));
+                unsafeAtomicAdd(rho + node, R(w[k]));
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
