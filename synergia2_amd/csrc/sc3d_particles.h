@@ -62,11 +62,10 @@ void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int6
                  int gy, int gz, const DomainRec* dom, SortBuffers& b, hipStream_t st);
 void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, const int32_t* perm,
                     double* scratch, uint8_t* smask, const DomainRec* dom, hipStream_t st);
-// Deposit: local (k_deposit_tile): windows of the bunch storage through an
-// LDS node tile of each window's cell box (the storage is cell-sorted at
-// every reorder); else (k_deposit): through the permutation `perm` of this
-// step's sort, compensated run sums in FP32.  FP32: unit weights; then
-// k_rho_peak records the density peak in the domain record.
+// Deposit (k_deposit_tile) of windows through an LDS node tile of each
+// window's cell box; local: windows of the bunch storage (cell-sorted at every
+// reorder), else of the permutation `perm` of this step's sort.  FP32: unit
+// weights; then k_rho_peak records the density peak in the domain record.
 template <typename R>
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
                     const int32_t* perm, bool local, int64_t n, int gx, int gy, int gz,

@@ -512,18 +512,12 @@ __device__ __forceinline__ int64_t count_at(int d, int64_t b, int nblk)
 // wavefront scans, instead of LDS permutes: rows of 16 lanes; a lane with no
 // source lane, or in a row outside ROW_MASK, returns `old`.
 constexpr int kDppRowShr = 0x110;  // + n: from lane - n of the same row
-constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;  // from lane + 1 / lane - 1
 constexpr int kDppRowBcast15 = 0x142;  // lane 15 of each row to the next row
 constexpr int kDppRowBcast31 = 0x143;  // lane 31 to rows 2 and 3
 template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ int dpp_move(int old, int v)
 {
     return __builtin_amdgcn_update_dpp(old, v, CTRL, ROW_MASK, 0xf, false);
-}
-template <int CTRL, int ROW_MASK = 0xf>
-__device__ __forceinline__ float dpp_move(float old, float v)
-{
-    return __int_as_float(dpp_move<CTRL, ROW_MASK>(__float_as_int(old), __float_as_int(v)));
 }
 template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ double dpp_move(double old, double v)
@@ -813,289 +807,17 @@ __global__ void k_fill(R* __restrict__ p, int64_t n, R v)
 // written only if 0 < idx < g-1 in all three axes (ingrid, :21-30).
 // Target: the G octant of rho2 (zyx, gx fastest).
 //
-// Through the sort permutation (k_deposit, used when the storage is never
-// reordered): the eight corner weights are summed over runs of equal cell
-// keys before any global atomic.  Every lane takes K consecutive particles
-// of the cell-sorted order and sums its own runs in order; a run that
-// starts and ends inside the lane is emitted at once.  The lanes' trailing runs are
-// then summed across lanes by one segmented inclusive scan (a segment
-// continues through lanes that hold a single run of the same key), and the
-// total reaching a lane whose leading run has that key is carried into it.
-// Every run is emitted once, by the lane where it ends.  Any particle order
-// is correct; a cell-sorted order gives about one run per cell and
-// wavefront.  Lanes past n and particles that are masked out or off the
-// grid break runs and add nothing.
-//
 // Precision form (FP32 grid): the cell index and offsets come from the FP64
-// coordinates as above; the weights are unit charge weights aox*aoy*aoz
-// (left to right) rounded to FP32, and all run sums are compensated FP32
-// (TwoSum: a sum and its rounding error, combined error-free), so a run's
-// total is its exact sum rounded once.  The physical weight w0 and the
-// unit-peak scale return in FP64 at the kick.
+// coordinates as above and the weights are unit charge weights aox*aoy*aoz;
+// the physical weight w0 and the unit-peak scale return in FP64 at the kick.
 // ---------------------------------------------------------------------------
-
-__device__ __forceinline__ void two_sum(float a, float b, float& s, float& e)
-{
-    s = a + b;
-    const float bb = s - a;
-    e = (a - (s - bb)) + (b - bb);
-}
-
-// Eight corner sums: FP64 plain, FP32 compensated.
-template <typename R> struct CornerSums;
-template <> struct CornerSums<double> {
-    double w[8];
-    __device__ __forceinline__ void add(const CornerSums& o)
-    {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) w[c] += o.w[c];
-    }
-    template <int CTRL, int ROW_MASK = 0xf> __device__ __forceinline__ CornerSums moved() const
-    {
-        CornerSums o;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) o.w[c] = dpp_move<CTRL, ROW_MASK>(0.0, w[c]);
-        return o;
-    }
-    __device__ __forceinline__ double total(int c) const { return w[c]; }
-};
-template <> struct CornerSums<float> {
-    float w[8], e[8];
-    __device__ __forceinline__ void add(const CornerSums& o)
-    {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            float t, err;
-            two_sum(w[c], o.w[c], t, err);
-            w[c] = t;
-            e[c] = (e[c] + o.e[c]) + err;
-        }
-    }
-    template <int CTRL, int ROW_MASK = 0xf> __device__ __forceinline__ CornerSums moved() const
-    {
-        CornerSums o;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            o.w[c] = dpp_move<CTRL, ROW_MASK>(0.0f, w[c]);
-            o.e[c] = dpp_move<CTRL, ROW_MASK>(0.0f, e[c]);
-        }
-        return o;
-    }
-    __device__ __forceinline__ float total(int c) const { return w[c] + e[c]; }
-};
-
-// The corner weights of one particle (ok: on the grid; else zeros).
-template <typename R>
-__device__ __forceinline__ CornerSums<R> corner_weights(bool ok, double ox, double oy, double oz,
-                                                        double w0)
-{
-    CornerSums<R> a;
-    if constexpr (sizeof(R) == sizeof(double)) {
-        const double aox = 1.0 - ox, aoy = 1.0 - oy, aoz = 1.0 - oz;
-        a.w[0] = w0 * aox * aoy * aoz;
-        a.w[1] = w0 * ox * aoy * aoz;
-        a.w[2] = w0 * aox * oy * aoz;
-        a.w[3] = w0 * ox * oy * aoz;
-        a.w[4] = w0 * aox * aoy * oz;
-        a.w[5] = w0 * ox * aoy * oz;
-        a.w[6] = w0 * aox * oy * oz;
-        a.w[7] = w0 * ox * oy * oz;
-    } else {
-        const float fx = float(ox), fy = float(oy), fz = float(oz);
-        const float ax = float(1.0 - ox), ay = float(1.0 - oy), az = float(1.0 - oz);
-        a.w[0] = ax * ay * az;
-        a.w[1] = fx * ay * az;
-        a.w[2] = ax * fy * az;
-        a.w[3] = fx * fy * az;
-        a.w[4] = ax * ay * fz;
-        a.w[5] = fx * ay * fz;
-        a.w[6] = ax * fy * fz;
-        a.w[7] = fx * fy * fz;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) a.e[c] = 0.0f;
-    }
-    if (!ok) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) a.w[c] = R(0);
-    }
-    return a;
-}
-
-// Adds one run's sums to the interior corners of cell `key`.
-template <typename R>
-__device__ __forceinline__ void add_run(R* __restrict__ rho, int key, const CornerSums<R>& a,
-                                        int gx, int gy, int gz)
-{
-    const int ix = key % gx, r = key / gx;
-    const int iy = r % gy, iz = r / gy;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const int cx = ix + (c & 1), cy = iy + ((c >> 1) & 1), cz = iz + (c >> 2);
-        if (cx > 0 && cx < gx - 1 && cy > 0 && cy < gy - 1 && cz > 0 && cz < gz - 1)
-            unsafeAtomicAdd(rho + (int64_t(cz) * gy + cy) * gx + cx, R(a.total(c)));
-    }
-}
-
-// The runs of one lane's K consecutive particles of a cell-sorted order and
-// the wavefront's combination (see above).  key[q] < 0 marks particles that
-// add nothing; those keys must differ from each other and from the keys of
-// every other lane of the wavefront.
-// Run totals go to `emit(key, sums, q_last)`, q_last = the lane index of the
-// run's last particle in this lane (K-1 for a run that goes on into the next
-// lane or wavefront).
-template <typename R> struct AtomicRuns {
-    R* __restrict__ rho;
-    int gx, gy, gz;
-    __device__ __forceinline__ void operator()(int key, const CornerSums<R>& a, int) const
-    {
-        add_run<R>(rho, key, a, gx, gy, gz);
-    }
-};
-
-// One step of the segmented scan: add the partial sum the lane move brings
-// when it comes from the same segment.
-template <int CTRL, int ROW_MASK, typename R>
-__device__ __forceinline__ void scan_step(CornerSums<R>& cur, int seg)
-{
-    const int seg_from = dpp_move<CTRL, ROW_MASK>(-1, seg);
-    const CornerSums<R> up = cur.template moved<CTRL, ROW_MASK>();
-    if (seg_from == seg) cur.add(up);
-}
-
-template <typename R, int K, typename Emit>
-__device__ __forceinline__ void deposit_runs(const int (&key)[K], const double (&ox)[K],
-                                             const double (&oy)[K], const double (&oz)[K],
-                                             double w0, const Emit& emit)
-{
-    const int lane = threadIdx.x & 63;
-    const uint64_t le_mask = (lane == 63) ? ~0ull : ((1ull << (lane + 1)) - 1);
-    // runs inside the lane: the leading run (head), the trailing run (cur at
-    // the end); runs in between are added at once
-    CornerSums<R> cur, head;
-    int cur_key = 0, head_key = 0, cur_start = 0, head_last = K - 1;
-    bool single = true;
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const CornerSums<R> p = corner_weights<R>(key[q] >= 0, ox[q], oy[q], oz[q], w0);
-        if (q == 0) {
-            cur = p;
-            cur_key = key[q];
-        } else if (key[q] == cur_key) {
-            cur.add(p);
-        } else {
-            if (cur_start == 0) {
-                head = cur;
-                head_key = cur_key;
-                head_last = q - 1;
-                single = false;
-            } else if (cur_key >= 0) {
-                emit(cur_key, cur, q - 1);
-            }
-            cur = p;
-            cur_key = key[q];
-            cur_start = q;
-        }
-    }
-    if (single) head_key = cur_key;
-    // trailing runs across lanes: segmented inclusive scan (every lane takes
-    // part in every lane move: a move must never run under a divergent exec
-    // mask).  seg >= 1 numbers the segments; a lane adds a moved partial sum
-    // only when it comes from its own segment (-1 marks no source lane).
-    const int prev_tail = dpp_move<kDppWaveShr1>(0, cur_key);
-    const bool start = lane == 0 || !single || prev_tail != cur_key;
-    const int seg = __popcll(__ballot(start) & le_mask);
-    // within rows of 16 lanes: from lane - 1, - 2, - 4, - 8 of the row
-    scan_step<kDppRowShr + 1, 0xf>(cur, seg);
-    scan_step<kDppRowShr + 2, 0xf>(cur, seg);
-    scan_step<kDppRowShr + 4, 0xf>(cur, seg);
-    scan_step<kDppRowShr + 8, 0xf>(cur, seg);
-    // across rows: lane 15 into row 1 and lane 47 into row 3, then lane 31
-    // (by now the sum through lane 31) into rows 2 and 3
-    scan_step<kDppRowBcast15, 0xa>(cur, seg);
-    scan_step<kDppRowBcast31, 0xc>(cur, seg);
-    // the total of the previous lane's trailing run continues this lane's
-    // leading run when the keys agree
-    const CornerSums<R> carry = cur.template moved<kDppWaveShr1>();
-    const int next_head = dpp_move<kDppWaveShl1>(0, head_key);
-    if (!single && head_key >= 0) {
-        if (lane > 0 && prev_tail == head_key) head.add(carry);
-        emit(head_key, head, head_last);
-    }
-    if (cur_key >= 0 && (lane == 63 || next_head != cur_key)) emit(cur_key, cur, K - 1);
-}
-
-// Deposit through the sort permutation of this step (every apply sorts;
-// used when the bunch storage is never reordered, sort_period 0).
-template <typename R, int K>
-__global__ __launch_bounds__(kThreads) void k_deposit(const double* __restrict__ parts,
-                                                      int64_t stride,
-                                                      const uint8_t* __restrict__ masks,
-                                                      const int32_t* __restrict__ perm_in,
-                                                      int64_t n, int gx, int gy, int gz,
-                                                      const DomainRec* __restrict__ dom,
-                                                      R* __restrict__ rho)
-{
-    if (dom->error) return;
-    const int32_t* __restrict__ perm = perm_in;
-    const double lx = dom->left[0], ly = dom->left[1], lz = dom->left[2];
-    const double ihx = dom->inv_h[0], ihy = dom->inv_h[1], ihz = dom->inv_h[2];
-    const int lane = threadIdx.x & 63;
-    // this lane's K consecutive positions of the cell-sorted order
-    const int64_t j0 = (blockIdx.x * int64_t(kThreads) + threadIdx.x) * K;
-    int64_t idx[K];
-    if (perm && j0 + K <= n && K % 4 == 0) {
-#pragma unroll
-        for (int v = 0; v < K / 4; ++v) {
-            const int4 p4 = *reinterpret_cast<const int4*>(perm + j0 + 4 * v);
-            idx[4 * v] = p4.x;
-            idx[4 * v + 1] = p4.y;
-            idx[4 * v + 2] = p4.z;
-            idx[4 * v + 3] = p4.w;
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < K; ++q) {
-            const int64_t j = j0 + q;
-            idx[q] = j < n ? (perm ? int64_t(perm[j]) : j) : -1;
-        }
-    }
-    double X[K], Y[K], Z[K];
-    bool M[K];
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        const int64_t j = j0 + q;
-        if (j < n && (idx[q] < 0 || idx[q] >= n)) idx[q] = j;  // perm is a permutation of [0, n)
-        M[q] = false;
-        X[q] = Y[q] = Z[q] = 0.0;
-        if (idx[q] >= 0) {
-            M[q] = masks[idx[q]] != 0;
-            X[q] = parts[idx[q]];
-            Y[q] = parts[idx[q] + 2 * stride];
-            Z[q] = parts[idx[q] + 4 * stride];
-        }
-    }
-    int key[K];
-    double ox[K], oy[K], oz[K];
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-        ox[q] = oy[q] = oz[q] = 0.0;
-        key[q] = -1 - (lane * K + q);  // off-grid particles: singletons
-        if (M[q]) {
-            const int ix = cell_index(X[q], lx, ihx, ox[q]);
-            const int iy = cell_index(Y[q], ly, ihy, oy[q]);
-            const int iz = cell_index(Z[q], lz, ihz, oz[q]);
-            if (ix >= 0 && ix <= gx - 2 && iy >= 0 && iy <= gy - 2 && iz >= 0 && iz <= gz - 2)
-                key[q] = (iz * gy + iy) * gx + ix;
-        }
-    }
-    deposit_runs<R, K>(key, ox, oy, oz, dom->w0, AtomicRuns<R>{rho, gx, gy, gz});
-}
 
 // Deposit in windows of the bunch storage through an LDS node tile.  The
 // storage is cell-sorted at every reorder (sort_period applies) and
-// particles move a few cells per step, so kTileWindow consecutive slots stay
-// a compact group of cells.  A block takes one window, each thread four
-// consecutive slots; the block reduces the window's cell bounding box, clears
+// particles move a few cells per step, so consecutive slots stay a compact
+// group of cells; PERM (storage never reordered): consecutive entries of this
+// apply's sort permutation.  A block takes one window of 256 PER slots, each
+// thread PER consecutive ones; the block reduces the window's cell bounding box, clears
 // that box of nodes in LDS (up to kTileNodes FP64 nodes), and every particle
 // adds its eight corner weights there with LDS FP64 atomics -- the corners of
 // a thread's consecutive particles in one cell summed in registers first,
@@ -1103,7 +825,7 @@ __global__ __launch_bounds__(kThreads) void k_deposit(const double* __restrict__
 // different nodes at a time.  The block then adds the box's non-zero
 // interior nodes to rho with global atomics (no sort, no scan, no run list).
 // A window whose box does not fit gives each wavefront a quarter of the
-// tile for the box of its own 256 particles (no block barrier: LDS
+// tile for the box of its own particles (no block barrier: LDS
 // operations of one wavefront complete in order); a wavefront whose box does
 // not fit either sums its corners in a direct-mapped FP64 cache of nodes in
 // its quarter (a crowded node of a scattered storage then takes one add per
@@ -1138,8 +860,6 @@ __global__ __launch_bounds__(kThreads) void k_deposit(const double* __restrict__
 // (about four runs a thread late in the sort period; then the LDS atomics and
 // the four blocks a CU holds are the limit).
 constexpr int kTileThreads = 256;
-constexpr int kTilePer = 4;                             // consecutive slots per thread
-constexpr int kTileWindow = kTileThreads * kTilePer;    // slots per block
 constexpr int kTileNodes = 4096;                        // FP64 nodes of the LDS tile (32 KiB)
 constexpr int kTileTailDiv = 8;                         // 1/8 of the windows rotated first
 constexpr int kTileWaves = kTileThreads / 64;
@@ -1257,10 +977,11 @@ __device__ __forceinline__ void tile_flush(const double* tile, int nodes, int fi
     }
 }
 
-template <typename R>
+template <typename R, int PER, bool PERM>
 __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     const double* __restrict__ parts, int64_t stride, const uint8_t* __restrict__ masks,
-    int64_t n, int gx, int gy, int gz, const DomainRec* __restrict__ dom, R* __restrict__ rho)
+    const int32_t* __restrict__ perm, int64_t n, int gx, int gy, int gz,
+    const DomainRec* __restrict__ dom, R* __restrict__ rho)
 {
     __shared__ double tile[kTileNodes];
     __shared__ int box[kTileWaves][6];
@@ -1274,17 +995,18 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     // the last eighth of the windows (one tail of the bunch) first
     const int nb = int(gridDim.x), tail = nb / kTileTailDiv;
     const int blk = (int(blockIdx.x) + nb - tail) % nb;
-    const int64_t base = int64_t(blk) * kTileWindow + int64_t(t) * kTilePer;
-    int ix[kTilePer], iy[kTilePer], iz[kTilePer];
-    double ox[kTilePer], oy[kTilePer], oz[kTilePer];
-    bool ok[kTilePer];
+    const int64_t base = int64_t(blk) * (kTileThreads * PER) + int64_t(t) * PER;
+    int ix[PER], iy[PER], iz[PER];
+    double ox[PER], oy[PER], oz[PER];
+    bool ok[PER];
     int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {-1, -1, -1};
 #pragma unroll
-    for (int q = 0; q < kTilePer; ++q) {
-        const int64_t j = base + q;
+    for (int q = 0; q < PER; ++q) {
+        int64_t j = base + q;
         double x = 0.0, y = 0.0, z = 0.0;
         bool m = false;
         if (j < n) {
+            if (PERM) j = perm[j];
             m = masks[j] != 0;
             x = parts[j];
             y = parts[j + 2 * stride];
@@ -1365,7 +1087,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int q = 0; q < kTilePer; ++q) {
+    for (int q = 0; q < PER; ++q) {
         if (!ok[q]) continue;
         double w[8];
         lc.weights(w0, ox[q], oy[q], oz[q], w);
@@ -2043,38 +1765,28 @@ void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, co
                        perm, n, scratch, smask, dom);
 }
 
-// Particles per lane of the deposit: 4 on dense bunches, 2 on sparse ones.
-// Measured (deposit phase, us): 4e6 particles on 64x64x128 (7.6 per cell)
-// FP64 K=4 72, K=2 74, K=8 99; FP32 K=4 84, K=2 86.  1.6e7 on 128x128x256
-// (3.8 per cell) FP32 K=4 317, K=2 264, K=8 421; FP64 K=4 324, K=2 284.
-// With few particles per cell most lanes end runs inside their K particles,
-// and those additions run under divergent masks.
-template <typename R>
-static void launch_deposit_k(const double* parts, int64_t stride, const uint8_t* masks,
-                             const int32_t* perm, int64_t n, int gx, int gy, int gz,
-                             DomainRec* dom, R* rho, hipStream_t st)
+template <typename R, bool PERM>
+static void launch_deposit_tiles(const double* parts, int64_t stride, const uint8_t* masks,
+                                 const int32_t* perm, int64_t n, int gx, int gy, int gz,
+                                 DomainRec* dom, R* rho, hipStream_t st)
 {
-    const int64_t G = int64_t(gx) * gy * gz;
-    const int K = n >= 6 * G ? 4 : 2;
-    const int64_t nb = (n + int64_t(kThreads) * K - 1) / (int64_t(kThreads) * K);
-    if (nb < 1) return;
-    if (K == 4)
-        hipLaunchKernelGGL((k_deposit<R, 4>), dim3(unsigned(nb)), dim3(kThreads), 0, st, parts,
-                           stride, masks, perm, n, gx, gy, gz, dom, rho);
+    auto launch = [&](auto kernel, int per) {
+        const int64_t win = kTileThreads * int64_t(per), nb = (n + win - 1) / win;
+        if (nb < 1) return;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(nb)), dim3(kTileThreads), 0, st, parts, stride,
+                           masks, perm, n, gx, gy, gz, dom, rho);
+    };
+    // Slots per thread: fewer where the windows would leave CUs idle (deposit
+    // phase at 1 / 2 / 4 slots, us: 1e4 particles 8.6 / 9.8 / 14.9, 1e5 8.4 / 9.1
+    // / 11.6 on 32x32x64; 4e5 on 64x64x128 14.8 / 12.6 / 15.5; 1e6 23.4 / 20.6 /
+    // 19.9); one through a permutation, whose random reads want the wavefronts
+    // (2e6 122 / 125 / 127, 4e6 266 / 273 / 279).
+    if (PERM || n < 250000)
+        launch(k_deposit_tile<R, 1, PERM>, 1);
+    else if (n < 750000)
+        launch(k_deposit_tile<R, 2, false>, 2);
     else
-        hipLaunchKernelGGL((k_deposit<R, 2>), dim3(unsigned(nb)), dim3(kThreads), 0, st, parts,
-                           stride, masks, perm, n, gx, gy, gz, dom, rho);
-}
-
-template <typename R>
-static void launch_deposit_local(const double* parts, int64_t stride, const uint8_t* masks,
-                                 int64_t n, int gx, int gy, int gz, DomainRec* dom, R* rho,
-                                 hipStream_t st)
-{
-    const int64_t nb = (n + kTileWindow - 1) / kTileWindow;
-    if (nb < 1) return;
-    hipLaunchKernelGGL(k_deposit_tile<R>, dim3(unsigned(nb)), dim3(kTileThreads), 0, st, parts,
-                       stride, masks, n, gx, gy, gz, dom, rho);
+        launch(k_deposit_tile<R, 4, false>, 4);
 }
 
 template <typename R>
@@ -2083,9 +1795,9 @@ void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
                     DomainRec* dom, R* rho, hipStream_t st)
 {
     if (local)
-        launch_deposit_local<R>(parts, stride, masks, n, gx, gy, gz, dom, rho, st);
+        launch_deposit_tiles<R, false>(parts, stride, masks, nullptr, n, gx, gy, gz, dom, rho, st);
     else
-        launch_deposit_k<R>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
+        launch_deposit_tiles<R, true>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
 }
 
 template <>
@@ -2094,9 +1806,9 @@ void launch_deposit<float>(const double* parts, int64_t stride, const uint8_t* m
                            DomainRec* dom, float* rho, hipStream_t st)
 {
     if (local)
-        launch_deposit_local<float>(parts, stride, masks, n, gx, gy, gz, dom, rho, st);
+        launch_deposit_tiles<float, false>(parts, stride, masks, nullptr, n, gx, gy, gz, dom, rho, st);
     else
-        launch_deposit_k<float>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
+        launch_deposit_tiles<float, true>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
     const int64_t G = int64_t(gx) * gy * gz;
     hipLaunchKernelGGL(k_rho_peak, dim3(grid_for(G / 8, 512)), dim3(kThreads), 0, st, rho, G, dom);
 }
