@@ -850,7 +850,6 @@ __global__ __launch_bounds__(kThreads) void k_green_x(
     const int nrows = (gz + 1) * (gy + 1);
     const int r0 = blockIdx.x * NL;
     const double hx = dom->h[0], hy = dom->h[1], hz = dom->h[2];
-    const double G000 = green_g000(green_fn, hx, hy, hz);
     for (int e = threadIdx.x; e < NL * (M + 1); e += kThreads) {
         int line = e / (M + 1), X = e % (M + 1);
         int r = r0 + line;
@@ -858,7 +857,7 @@ __global__ __launch_bounds__(kThreads) void k_green_x(
         if (r < nrows) {
             int Z = r / (gy + 1), Y = r - Z * (gy + 1);
             double x = X * hx, y = Y * hy, z = Z * hz;
-            v = green_value(green_fn, x, y, z, hz, G000);
+            v = green_value(green_fn, x, y, z, hx, hy, hz);
         }
         row[e] = T(v);
     }

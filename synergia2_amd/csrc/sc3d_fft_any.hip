@@ -1013,13 +1013,12 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_green_x(
     constexpr int W = any_rows_per<T2>();
     const int r0 = W * (int(blockIdx.x) * a.nl + q.line), r1 = W == 2 ? r0 + 1 : nrows;
     const double hx = dom->h[0], hy = dom->h[1], hz = dom->h[2];
-    const double G000 = green_g000(green_fn, hx, hy, hz);
     if (q.line >= 0) {
         T2* lb = m.buf + q.line * a.st;
         auto value = [&](int r, int x) -> T {
             if (r >= nrows) return T(0);
             const int Z = r / (gy + 1), Y = r - Z * (gy + 1);
-            return T(green_value(green_fn, x * hx, Y * hy, Z * hz, hz, G000));
+            return T(green_value(green_fn, x * hx, Y * hy, Z * hz, hx, hy, hz));
         };
         for (int x = q.j; x < Hx; x += a.tpl) {
             T2 c;

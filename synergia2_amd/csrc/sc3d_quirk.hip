@@ -195,18 +195,17 @@ __global__ __launch_bounds__(kThreads) void k_green_patch(
     if (dom->error) return;
     const double hx = dom->h[0], hy = dom->h[1], hz = dom->h[2];
     const int Dx = 2 * gx, Dy = 2 * gy, Dz = 2 * gz;
-    const double G000 = green_g000(green_fn, hx, hy, hz);
     for (int p = threadIdx.x; p < np; p += kThreads) {
         const GreenPatch P = patches[p];
         const int Z = P.t[0], Y = P.t[1], X = P.t[2];
         double sym = green_value(green_fn, min(X, Dx - X) * hx, min(Y, Dy - Y) * hy,
-                                 min(Z, Dz - Z) * hz, hz, G000);
+                                 min(Z, Dz - Z) * hz, hx, hy, hz);
         double val = 0.0;
         if (P.s[0] >= 0) {
             const int iz = P.s[0], iy = P.s[1], ix = P.s[2];
             // linear: z folded as alg_g2_linear does (:280); pointlike: iz <= gz
             const double z = (green_fn == SC3D_GREEN_LINEAR && iz > gz) ? (Dz - iz) * hz : iz * hz;
-            val = green_value(green_fn, ix * hx, iy * hy, z, hz, G000);
+            val = green_value(green_fn, ix * hx, iy * hy, z, hx, hy, hz);
         }
         dlt[p] = val - sym;
         tz[p] = Z;
@@ -268,16 +267,15 @@ __global__ __launch_bounds__(kThreads) void k_patch_values(
     if (p >= np) return;
     const double hx = dom->h[0], hy = dom->h[1], hz = dom->h[2];
     const int Dx = 2 * gx, Dy = 2 * gy, Dz = 2 * gz;
-    const double G000 = green_g000(green_fn, hx, hy, hz);
     const GreenPatch P = patches[p];
     const int Z = P.t[0], Y = P.t[1], X = P.t[2];
     const double sym = green_value(green_fn, min(X, Dx - X) * hx, min(Y, Dy - Y) * hy,
-                                   min(Z, Dz - Z) * hz, hz, G000);
+                                   min(Z, Dz - Z) * hz, hx, hy, hz);
     double val = 0.0;
     if (P.s[0] >= 0) {
         const int iz = P.s[0], iy = P.s[1], ix = P.s[2];
         const double z = (green_fn == SC3D_GREEN_LINEAR && iz > gz) ? (Dz - iz) * hz : iz * hz;
-        val = green_value(green_fn, ix * hx, iy * hy, z, hz, G000);
+        val = green_value(green_fn, ix * hx, iy * hy, z, hx, hy, hz);
     }
     C[(int64_t(Z) * Dy + Y) * Dx + X] = R(val - sym);
 }
