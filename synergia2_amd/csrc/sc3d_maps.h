@@ -60,6 +60,18 @@ constexpr int kYoshidaDrifts = 10;
 constexpr int kYoshidaDriftOrder[kYoshidaDrifts] = {0, 1, 1, 2, 3, 3, 2, 1, 1, 0};
 constexpr int kYoshidaKickOrder[kYoshidaDrifts] = {0, 1, 0, 2, 3, 2, 0, 1, 0, 0};  // 9 used
 
+// The stages one after the other, for the rolled loops.
+struct YoshidaStage {
+    double drift, kick;
+};
+constexpr YoshidaStage yoshida_stage(int q)
+{
+    return {kYoshidaDrift[kYoshidaDriftOrder[q]], kYoshidaKick[kYoshidaKickOrder[q]]};
+}
+constexpr YoshidaStage kYoshidaStages[kYoshidaDrifts] = {
+    yoshida_stage(0), yoshida_stage(1), yoshida_stage(2), yoshida_stage(3), yoshida_stage(4),
+    yoshida_stage(5), yoshida_stage(6), yoshida_stage(7), yoshida_stage(8), yoshida_stage(9)};
+
 // General form; rolled, so that on the device it stays out of the way of the
 // fast form's registers (unrolled it set the maps kernels' count: 147 VGPRs).
 __host__ __device__ inline void yoshida6_quad(double& x, double& xp, double& y, double& yp,
@@ -72,11 +84,10 @@ __host__ __device__ inline void yoshida6_quad(double& x, double& xp, double& y, 
     for (int i = 0; i < steps; ++i) {
 #pragma nounroll
         for (int q = 0; q < kYoshidaDrifts; ++q) {
-            drift_unit(x, xp, y, yp, cdt, dpop, kYoshidaDrift[kYoshidaDriftOrder[q]] * step_length,
-                       reference_momentum, m, sub);
+            const YoshidaStage g = kYoshidaStages[q];
+            drift_unit(x, xp, y, yp, cdt, dpop, g.drift * step_length, reference_momentum, m, sub);
             if (q == kYoshidaDrifts - 1) break;
-            const double d = kYoshidaKick[kYoshidaKickOrder[q]];
-            const double kL[2] = {d * step_strength[0], d * step_strength[1]};
+            const double kL[2] = {g.kick * step_strength[0], g.kick * step_strength[1]};
             thin_quadrupole_unit(x, xp, y, yp, kL);
         }
     }
@@ -145,9 +156,10 @@ struct MapProgram {
 //      ulp: that is its seed, and s/(2 |l| C) the slope, for one residual step.
 //      Signed by l, so no separate sign multiplication.
 // The last step needs |l| C / s accurate to a few ulp, so a in [1/2, 2] (no
-// cancellation) and 1/beta^2 away from 1 (at 1 and |l| near a power of two
-// D2/beta^2 comes next to a power of four, where one residual step cannot
-// decide the rounding); a particle or slice outside that takes drift_unit.
+// cancellation; a particle outside takes drift_unit) and 1/beta^2 away from 1
+// (at 1 and |l| near a power of two D2/beta^2 comes next to a power of four,
+// where one residual step cannot decide the rounding; there the path length
+// has a square root of its own).
 // Measured (4e6 particles, mean over the 10 steps of an O-F-O-D cell, 6
 // quadrupole slices among them): maps pass 266 -> 178 us, kick with maps fused
 // (whole step) 449 -> 364 us; a step of drifts alone stays at 54 us, its
@@ -156,6 +168,7 @@ struct MapProgram {
 // took the kernel to 156 VGPRs.
 // ---------------------------------------------------------------------------
 constexpr int32_t kHighOfHalf = 0x3fe00000;  // high word of 0.5
+constexpr double kNearLight = 1.0 + 1.0e-6;  // 1/beta^2, see above
 
 struct FastDrift {
     double dp2, ibeta2, c, half_rc;  // (1+dp/p)^2, 1/beta^2, C, 0.5 / C
@@ -164,11 +177,11 @@ struct FastDrift {
 };
 
 // Whether the slices of a program may take the fast form (the range keeps
-// every residual of the path length normal; skew kicks take the general form).
+// every residual of the path length normal).
 __device__ __forceinline__ bool fast_slice(const PreparedSlice& s)
 {
     const double l = fabs(s.length);
-    return l > 1.0e-60 && l < 1.0e60 && s.k[1] == 0.0;
+    return (l > 1.0e-60 && l < 1.0e60) || (s.kind == SC3D_MAP_DRIFT && l == 0.0);
 }
 
 __device__ __forceinline__ bool fast_begin(FastDrift& f, double dpop, double ref_p, double m)
@@ -182,7 +195,14 @@ __device__ __forceinline__ bool fast_begin(FastDrift& f, double dpop, double ref
     f.half_rc = 0.5 / f.c;
     f.a_low = INT32_MAX;
     f.ones = 0u;
-    return dp > 0.0 && f.dp2 <= 2.0 && f.ibeta2 > 1.0 + 1.0e-6 && f.ibeta2 < 1.0e12;
+    return dp > 0.0 && f.dp2 <= 2.0 && f.ibeta2 >= 1.0 && f.ibeta2 < 1.0e12;
+}
+
+__device__ __forceinline__ double fast_a(FastDrift& f, double xp, double yp)
+{
+    const double a = f.dp2 - xp * xp - yp * yp;
+    f.a_low = min(f.a_low, int32_t(__double_as_longlong(a) >> 32));
+    return a;
 }
 
 __device__ __forceinline__ bool fast_held(const FastDrift& f)
@@ -190,13 +210,14 @@ __device__ __forceinline__ bool fast_held(const FastDrift& f)
     return f.a_low >= kHighOfHalf && f.ones != 0xffffffffu;
 }
 
-// drift_unit over length l (l2 = l*l); kl ~ l C, hl ~ 1 / (2 l C)
+// drift_unit over length l (l2 = l*l); kl ~ l C, hl ~ 1 / (2 l C).  OWN_ROOT:
+// the path length by a square root of its own (kl, hl unused).
+template <bool OWN_ROOT>
 __device__ __forceinline__ void fast_drift(FastDrift& f, double& x, double xp, double& y,
                                            double yp, double& cdt, double l, double l2, double kl,
                                            double hl, double ref_cdt)
 {
-    const double a = f.dp2 - xp * xp - yp * yp;
-    f.a_low = min(f.a_low, int32_t(__double_as_longlong(a) >> 32));
+    const double a = fast_a(f, xp, yp);
     const double yr = rsqrt_near(a);
     const double s = sqrt_from(a, yr);
     f.ones = max(f.ones, uint32_t(__double_as_longlong(s)));
@@ -205,8 +226,13 @@ __device__ __forceinline__ void fast_drift(FastDrift& f, double& x, double xp, d
     const double lypr = yp * l * inv_npz;
     const double D2 = lxpr * lxpr + l2 + lypr * lypr;
     const double A = D2 * f.ibeta2;
-    const double t = kl * inv_npz;
-    const double path = __builtin_fma(__builtin_fma(-t, t, A), s * hl, t);
+    double path;
+    if (OWN_ROOT) {
+        path = __builtin_copysign(sqrt_normal(A), l);
+    } else {
+        const double t = kl * inv_npz;
+        path = __builtin_fma(__builtin_fma(-t, t, A), s * hl, t);
+    }
     x = x + lxpr;
     y = y + lypr;
     cdt = cdt + path - ref_cdt;
@@ -221,26 +247,15 @@ __device__ __forceinline__ double uniform_f64(double v)
     return __longlong_as_double((long long)((uint64_t(hi) << 32) | lo));
 }
 
-// thin_quadrupole_unit with a zero skew strength (ks = +-0: the products with
-// it are exact, so a fused multiply-add rounds as the product and the sum do)
-__device__ __forceinline__ void fast_kick(double x, double& xp, double y, double& yp, double k,
-                                          double ks)
+// yoshida6_quad by fast drifts.  With no skew strength its products are +-0,
+// which a finite sum does not feel, and a coordinate that is not finite makes a
+// so as well (the general form).
+__device__ __forceinline__ void fast_quad(FastDrift& f, const PreparedSlice& s, double& x,
+                                          double& xp, double& y, double& yp, double& cdt)
 {
-    xp = __builtin_fma(ks, y, xp - k * x);
-    yp = __builtin_fma(ks, x, yp + k * y);
-}
-
-__device__ __forceinline__ void fast_slice_apply(FastDrift& f, const PreparedSlice& s, double& x,
-                                                 double& xp, double& y, double& yp, double& cdt)
-{
-    if (s.kind == SC3D_MAP_DRIFT) {
-        const double l = s.length;
-        fast_drift(f, x, xp, y, yp, cdt, l, l * l, l * f.c, f.half_rc / l, s.ref_cdt);
-        return;
-    }
     const double r = f.half_rc / s.length, kc = f.c * s.length;
     const double sub = uniform_f64(s.ref_cdt * 0.1);
-    double l[4], l2[4], kl[4], hl[4], k[4], ks[4];
+    double l[4], l2[4], kl[4], hl[4], k[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         l[j] = uniform_f64(kYoshidaDrift[j] * s.length);
@@ -248,15 +263,59 @@ __device__ __forceinline__ void fast_slice_apply(FastDrift& f, const PreparedSli
         kl[j] = kYoshidaDrift[j] * kc;
         hl[j] = (1.0 / kYoshidaDrift[j]) * r;
         k[j] = uniform_f64(kYoshidaKick[j] * s.k[0]);
-        ks[j] = uniform_f64(kYoshidaKick[j] * s.k[1]);
     }
     for (int i = 0; i < s.steps; ++i) {
 #pragma unroll
         for (int q = 0; q < kYoshidaDrifts; ++q) {
             const int j = kYoshidaDriftOrder[q], n = kYoshidaKickOrder[q];
-            fast_drift(f, x, xp, y, yp, cdt, l[j], l2[j], kl[j], hl[j], sub);
-            if (q < kYoshidaDrifts - 1) fast_kick(x, xp, y, yp, k[n], ks[n]);
+            fast_drift<false>(f, x, xp, y, yp, cdt, l[j], l2[j], kl[j], hl[j], sub);
+            if (q < kYoshidaDrifts - 1) {
+                xp = xp - k[n] * x;
+                yp = yp + k[n] * y;
+            }
         }
+    }
+}
+
+// The same with a skew strength, and next to the speed of light; rolled: a
+// second unrolled form does not fit the 128 registers (740 us where
+// the unrolled one takes 505 and the general one 1000; 4e6 particles, O-F-O-D).
+__device__ __forceinline__ void fast_quad_rolled(FastDrift& f, const PreparedSlice& s, double& x,
+                                                 double& xp, double& y, double& yp, double& cdt)
+{
+    const double sub = s.ref_cdt * 0.1;
+    for (int i = 0; i < s.steps; ++i) {
+#pragma nounroll
+        for (int q = 0; q < kYoshidaDrifts; ++q) {
+            const YoshidaStage g = kYoshidaStages[q];
+            const double l = uniform_f64(g.drift * s.length);
+            fast_drift<true>(f, x, xp, y, yp, cdt, l, l * l, 0.0, 0.0, sub);
+            if (q == kYoshidaDrifts - 1) break;
+            const double kL[2] = {g.kick * s.k[0], g.kick * s.k[1]};
+            thin_quadrupole_unit(x, xp, y, yp, kL);
+        }
+    }
+}
+
+__device__ __forceinline__ void fast_slice_apply(FastDrift& f, const PreparedSlice& s, double& x,
+                                                 double& xp, double& y, double& yp, double& cdt)
+{
+    const bool rolled = f.ibeta2 <= kNearLight;
+    const double l = s.length;
+    if (s.kind == SC3D_MAP_DRIFT) {
+        if (l == 0.0) {
+            fast_a(f, xp, yp);
+            x = x + xp * l;
+            y = y + yp * l;
+            cdt = cdt + 0.0 - s.ref_cdt;
+        } else if (rolled)
+            fast_drift<true>(f, x, xp, y, yp, cdt, l, l * l, 0.0, 0.0, s.ref_cdt);
+        else
+            fast_drift<false>(f, x, xp, y, yp, cdt, l, l * l, l * f.c, f.half_rc / l, s.ref_cdt);
+    } else if (rolled || s.k[1] != 0.0) {
+        fast_quad_rolled(f, s, x, xp, y, yp, cdt);
+    } else {
+        fast_quad(f, s, x, xp, y, yp, cdt);
     }
 }
 
