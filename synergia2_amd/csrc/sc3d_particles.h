@@ -42,10 +42,9 @@ struct SortBuffers {
     int32_t* keysB;
     int32_t* valsA;
     int32_t* valsB;
-    int32_t* counts;  // 256 * tiles
-    int32_t* totals;  // 256
-    int32_t* sorted_keys;  // result views (point into A/B)
-    int32_t* perm;
+    int32_t* counts;  // 2048 * tiles of kSortTileItems
+    int32_t* totals;  // 2048
+    int32_t* perm;  // result view (points into A/B)
 };
 
 constexpr int kSortTileItems = 4096;
@@ -57,7 +56,6 @@ void launch_step_begin(StepCtl* ctl, hipStream_t st);
 // scheduled maps before the kick (the first step's first half-step)
 void launch_maps_sched(double* parts, int64_t stride, const uint8_t* masks, int64_t n,
                        const Sched& sc, hipStream_t st);
-int sort_passes(int64_t G);
 void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int64_t n, int gx,
                  int gy, int gz, const DomainRec* dom, SortBuffers& b, hipStream_t st);
 void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, const int32_t* perm,

@@ -442,39 +442,40 @@ __device__ __forceinline__ int32_t brick_key(int ix, int iy, int iz, int gx, int
     return (brick << (sx + sy + sz)) + cell;
 }
 
-__device__ __forceinline__ int32_t cell_key(const double* __restrict__ parts, int64_t stride,
-                                            const uint8_t* __restrict__ masks, int64_t i, int gx,
+__device__ __forceinline__ int32_t cell_key(bool active, double x, double y, double z, int gx,
                                             int gy, int gz, const DomainRec& d)
 {
     double o;
-    const int ix = cell_index(parts[i], d.left[0], d.inv_h[0], o);
-    const int iy = cell_index(parts[i + 2 * stride], d.left[1], d.inv_h[1], o);
-    const int iz = cell_index(parts[i + 4 * stride], d.left[2], d.inv_h[2], o);
-    const bool in = masks[i] && ix >= 0 && ix < gx - 1 && iy >= 0 && iy < gy - 1 && iz >= 0 &&
-                    iz < gz - 1;
-    return in ? brick_key(ix, iy, iz, gx, gy, gz) : gx * gy * gz;
+    int ix, iy, iz;
+    const bool in_x = grid_cell(x, d.left[0], d.inv_h[0], gx, ix, o);
+    const bool in_y = grid_cell(y, d.left[1], d.inv_h[1], gy, iy, o);
+    const bool in_z = grid_cell(z, d.left[2], d.inv_h[2], gz, iz, o);
+    const int32_t key = brick_key(ix, iy, iz, gx, gy, gz);
+    return (active & in_x & in_y & in_z) ? key : gx * gy * gz;
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort of (key, index): digits of `width` <= 8 bits, tiles
-// of 4096 items (256 lanes x 16 rounds).  In the scatter, equal digits inside
-// a wavefront are matched with `width` ballots, so ranks need one LDS update
-// per distinct digit per wavefront.
+// Stable LSD radix sort of (key, index): tiles of 256 lanes x ITEMS rounds,
+// digits of up to 8 bits, or of 9 where that takes fewer passes.  In
+// the scatter, equal digits inside a wavefront are matched with `width`
+// ballots, so ranks need one LDS update per distinct digit per wavefront.
 // ---------------------------------------------------------------------------
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kThreads * kSortItems;
 constexpr int kMaxDigitBits = 8;
-constexpr int kMaxBuckets = 1 << kMaxDigitBits;
+constexpr int kWideDigitBits = 9;
 
 // lanes of this wavefront holding the same digit (valid lanes only)
 __device__ __forceinline__ uint64_t match_digit(int d, bool valid, int width)
 {
-    uint64_t peers = __ballot(valid);
+    const uint64_t v = __ballot(valid);
+    uint32_t lo = uint32_t(v), hi = uint32_t(v >> 32);
+#pragma unroll 2
     for (int b = 0; b < width; ++b) {
-        const uint64_t m = __ballot((d >> b) & 1);
-        peers &= ((d >> b) & 1) ? m : ~m;
+        const int32_t bit = __builtin_amdgcn_sbfe(d, b, 1);  // 0 or -1
+        const uint64_t m = __ballot(bit);
+        lo &= ~(uint32_t(m) ^ uint32_t(bit));
+        hi &= ~(uint32_t(m >> 32) ^ uint32_t(bit));
     }
-    return peers;
+    return uint64_t(hi) << 32 | lo;
 }
 
 #ifndef SC3D_XCD_PART
@@ -586,44 +587,60 @@ __device__ __forceinline__ int32_t block_exclusive_scan(int32_t v, int32_t* wsum
 }
 
 // Histogram of one digit per tile.  Every lane first loads (or, with KEYS,
-// computes from the particles and stores) its 16 keys, so all loads of the
+// computes from the particles and stores) its keys, so all loads of the
 // tile are in flight together; each wavefront then counts its quarter of
 // the tile into its own LDS histogram, one update per distinct digit and
 // round (ballot match: after the first pass equal digits cluster), and the
-// four are summed.  KEYS fuses the key pass into pass 0.
-template <bool KEYS>
+// four are summed.  KEYS fuses the key pass into pass 0.  WIDTH: largest
+// digit width taken.
+template <bool KEYS, int ITEMS, int WIDTH>
 __global__ __launch_bounds__(kThreads) void k_radix_count(
     const double* __restrict__ parts, int64_t stride, const uint8_t* __restrict__ masks, int gx,
     int gy, int gz, int32_t* __restrict__ keys, int64_t n, int shift, int width,
     int32_t* __restrict__ counts, int nblk, const DomainRec* __restrict__ dom)
 {
     constexpr int kWaves = kThreads / 64;
-    constexpr int kWaveItems = kSortTile / kWaves;
-    __shared__ int32_t hist[kWaves][kMaxBuckets];
+    constexpr int kTile = kThreads * ITEMS;
+    constexpr int kWaveItems = kTile / kWaves;
+    constexpr int kPer = (1 << WIDTH) / kThreads;  // digits per thread
+    __shared__ int32_t hist[kWaves][1 << WIDTH];
     if (dom->error) return;
     const unsigned blk = part_block();
     if (blk >= unsigned(nblk)) return;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int nb = 1 << width;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) hist[w][t] = 0;
-    const int64_t base = int64_t(blk) * kSortTile + int64_t(wave) * kWaveItems;
-    int32_t kk[kSortItems];
+    for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) hist[w][q * kThreads + t] = 0;
+    const int64_t base = int64_t(blk) * kTile + int64_t(wave) * kWaveItems;
+    int32_t kk[ITEMS];
     if (KEYS) {
         const DomainRec d = *dom;
+        constexpr int kBatch = 4;  // particles loaded ahead (a lane past n reads the last one)
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
-            const int64_t i = base + r * 64 + lane;
-            kk[r] = i < n ? cell_key(parts, stride, masks, i, gx, gy, gz, d) : -1;
-        }
+        for (int r0 = 0; r0 < ITEMS; r0 += kBatch) {
+            double x[kBatch], y[kBatch], z[kBatch];
+            uint8_t m[kBatch];
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
-            const int64_t i = base + r * 64 + lane;
-            if (i < n) keys[i] = kk[r];
+            for (int j = 0; j < kBatch; ++j) {
+                const int64_t i = min(base + (r0 + j) * 64 + lane, n - 1);
+                x[j] = parts[i];
+                y[j] = parts[i + 2 * stride];
+                z[j] = parts[i + 4 * stride];
+                m[j] = masks[i];
+            }
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j) {
+                const int64_t i = base + (r0 + j) * 64 + lane;
+                const int32_t key = cell_key(m[j] != 0, x[j], y[j], z[j], gx, gy, gz, d);
+                kk[r0 + j] = i < n ? key : -1;
+                if (i < n) keys[i] = key;
+            }
         }
     } else {
 #pragma unroll
-        for (int r = 0; r < kSortItems; ++r) {
+        for (int r = 0; r < ITEMS; ++r) {
             const int64_t i = base + r * 64 + lane;
             kk[r] = i < n ? keys[i] : -1;  // keys are >= 0
         }
@@ -631,18 +648,21 @@ __global__ __launch_bounds__(kThreads) void k_radix_count(
     __syncthreads();
     const uint64_t lt_mask = (1ull << lane) - 1;
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) {
+    for (int r = 0; r < ITEMS; ++r) {
         const bool valid = kk[r] >= 0;
         const int dg = (kk[r] >> shift) & (nb - 1);
         const uint64_t peers = match_digit(dg, valid, width);
         if (valid && __popcll(peers & lt_mask) == 0) hist[wave][dg] += __popcll(peers);
     }
     __syncthreads();
-    if (t < nb) {
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int d = q * kThreads + t;
+        if (d >= nb) break;
         int32_t c = 0;
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) c += hist[w][t];
-        counts[count_at(t, blk, nblk)] = c;
+        for (int w = 0; w < kWaves; ++w) c += hist[w][d];
+        counts[count_at(d, blk, nblk)] = c;
     }
 }
 
@@ -672,8 +692,8 @@ __global__ __launch_bounds__(kThreads) void k_radix_scan(int32_t* __restrict__ c
     if (threadIdx.x == 0) totals[d] = total;
 }
 
-// Stable scatter of one tile (4096 items).  Wavefront w ranks the items
-// [1024w, 1024w + 1024) of the tile in 16 rounds of 64 with wave-private
+// Stable scatter of one tile.  Wavefront w ranks the w-th quarter of the
+// tile's items in ITEMS rounds of 64 with wave-private
 // digit counters (ballot match: rank among equal digits of the round, the
 // lowest lane of each digit group advances the counter), with no block
 // barrier inside the rounds.  The tile's digit counts come from the count
@@ -682,6 +702,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scan(int32_t* __restrict__ c
 // tile is written out in that order, so each digit's items of the tile form
 // one contiguous run in the output (positions as a per-item scatter would
 // give them).
+template <int ITEMS, int WIDTH>
 __global__ __launch_bounds__(kThreads) void k_radix_scatter(
     const int32_t* __restrict__ keys_in, const int32_t* __restrict__ vals_in, int64_t n,
     int shift, int width, const int32_t* __restrict__ counts, const int32_t* __restrict__ totals,
@@ -689,76 +710,94 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
     const DomainRec* dom)
 {
     constexpr int kWaves = kThreads / 64;
-    constexpr int kWaveItems = kSortTile / kWaves;
-    __shared__ int32_t base_d[kMaxBuckets];   // output position of the tile's first digit-d item
-    __shared__ int32_t start_d[kMaxBuckets];  // its position inside the tile
-    __shared__ int32_t wave_off[kWaves][kMaxBuckets];
+    constexpr int kTile = kThreads * ITEMS;
+    constexpr int kWaveItems = kTile / kWaves;
+    constexpr int kPer = (1 << WIDTH) / kThreads;  // digits per thread, consecutive
+    __shared__ int32_t delta[1 << WIDTH];  // output position of a digit's items less that in the tile
+    __shared__ int32_t wave_off[kWaves][1 << WIDTH];
     __shared__ int32_t wsum[2][kWaves];
-    __shared__ int32_t lkey[kSortTile];
-    __shared__ int32_t lval[kSortTile];
+    __shared__ int32_t lkey[kTile];
+    __shared__ int32_t lval[kTile];
     if (dom->error) return;
     const unsigned blk = part_block();
     if (blk >= unsigned(nblk)) return;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int nb = 1 << width;  // <= kMaxBuckets == kThreads: thread t owns digit t
-    const int64_t tile = int64_t(blk) * kSortTile;
-    const int nvalid = int(n - tile < kSortTile ? n - tile : kSortTile);
+    const int nb = 1 << width;
+    const int64_t tile = int64_t(blk) * kTile;
+    const int nvalid = int(n - tile < kTile ? n - tile : kTile);
+    // all of the tile's loads in flight together
+    int32_t kk[ITEMS], vv[ITEMS], rk[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const int64_t i = tile + int64_t(wave) * kWaveItems + r * 64 + lane;
+        kk[r] = i < n ? keys_in[i] : -1;  // keys are >= 0; -1 marks lanes past n
+        vv[r] = i < n ? (vals_in ? vals_in[i] : int32_t(i)) : 0;
+    }
     // digit totals -> exclusive prefix over digits (global digit bases);
     // this tile's digit counts -> local digit starts
-    const int32_t tot = t < nb ? totals[t] : 0;
-    int32_t cnt = 0, before = 0;
-    if (t < nb) {
-        before = counts[count_at(t, blk, nblk)];
-        const int32_t next = blk + 1 < unsigned(nblk) ? counts[count_at(t, blk + 1, nblk)] : tot;
-        cnt = next - before;
+    int32_t tot[kPer], cnt[kPer], before[kPer], tsum = 0, csum = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int d = t * kPer + q;
+        tot[q] = cnt[q] = before[q] = 0;
+        if (d < nb) {
+            tot[q] = totals[d];
+            before[q] = counts[count_at(d, blk, nblk)];
+            cnt[q] = (blk + 1 < unsigned(nblk) ? counts[count_at(d, blk + 1, nblk)] : tot[q]) -
+                     before[q];
+        }
+        tsum += tot[q];
+        csum += cnt[q];
     }
     int32_t all_n, tile_n;
-    const int32_t digit_base = block_exclusive_scan(tot, wsum[0], all_n);
-    const int32_t local_start = block_exclusive_scan(cnt, wsum[1], tile_n);
-    if (t < nb) {
-        base_d[t] = digit_base + before;
-        start_d[t] = local_start;
+    int32_t digit_base = block_exclusive_scan(tsum, wsum[0], all_n);
+    int32_t local_start = block_exclusive_scan(csum, wsum[1], tile_n);
+    int32_t start[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        start[q] = local_start;
+        delta[t * kPer + q] = digit_base + before[q] - local_start;
+        digit_base += tot[q];
+        local_start += cnt[q];
     }
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) wave_off[w][t] = 0;
+    for (int w = 0; w < kWaves; ++w)
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) wave_off[w][q * kThreads + t] = 0;
     __syncthreads();
     // ranking inside each wavefront's quarter of the tile
     const uint64_t lt_mask = (1ull << lane) - 1;
-    int32_t kk[kSortItems], vv[kSortItems], rk[kSortItems];
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) {
-        const int64_t i = tile + int64_t(wave) * kWaveItems + r * 64 + lane;
-        const bool valid = i < n;
-        const int32_t key = valid ? keys_in[i] : 0;
-        const int32_t val = valid ? (vals_in ? vals_in[i] : int32_t(i)) : 0;
-        const int dg = (key >> shift) & (nb - 1);
+    for (int r = 0; r < ITEMS; ++r) {
+        const bool valid = kk[r] >= 0;
+        const int dg = (kk[r] >> shift) & (nb - 1);
         const uint64_t peers = match_digit(dg, valid, width);
         const int rank = __popcll(peers & lt_mask);
         // every lane of a digit group reads the counter before its lowest
         // lane advances it (LDS operations of a wavefront complete in order)
         const int32_t seen = wave_off[wave][dg];
         if (valid && rank == 0) wave_off[wave][dg] = seen + __popcll(peers);
-        kk[r] = valid ? key : -1;
-        vv[r] = val;
         rk[r] = seen + rank;
     }
     __syncthreads();
-    if (t < nb) {  // exclusive prefix over wavefronts, per digit
-        int32_t acc = 0;
+    // the tile position of each wavefront's first item of a digit
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        int32_t acc = start[q];
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
-            const int32_t c = wave_off[w][t];
-            wave_off[w][t] = acc;
+            const int32_t c = wave_off[w][t * kPer + q];
+            wave_off[w][t * kPer + q] = acc;
             acc += c;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) {
-        if (kk[r] < 0) continue;  // keys are >= 0; -1 marks lanes past n
+    for (int r = 0; r < ITEMS; ++r) {
+        if (kk[r] < 0) continue;
         const int dg = (kk[r] >> shift) & (nb - 1);
-        const int lpos = start_d[dg] + wave_off[wave][dg] + rk[r];
-        if (lpos >= 0 && lpos < kSortTile) {  // always true for consistent counts
+        const int lpos = wave_off[wave][dg] + rk[r];
+        if (lpos >= 0 && lpos < kTile) {  // always true for consistent counts
             lkey[lpos] = kk[r];
             lval[lpos] = vv[r];
         }
@@ -767,7 +806,7 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
     for (int j = t; j < nvalid; j += kThreads) {
         const int32_t key = lkey[j];
         const int dg = (key >> shift) & (nb - 1);
-        const int64_t pos = int64_t(base_d[dg]) + (j - start_d[dg]);
+        const int64_t pos = int64_t(delta[dg]) + j;
         if (pos >= 0 && pos < n) {  // always true for consistent counts
             keys_out[pos] = key;
             vals_out[pos] = lval[j];
@@ -1703,28 +1742,18 @@ void launch_step_begin(StepCtl* ctl, hipStream_t st)
     hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, st, ctl);
 }
 
-int sort_passes(int64_t G)
+template <int ITEMS, int WIDTH>
+static void launch_sort_tiles(const double* parts, int64_t stride, const uint8_t* masks, int64_t n,
+                              int gx, int gy, int gz, const DomainRec* dom, SortBuffers& b,
+                              int bits, hipStream_t st)
 {
-    int bits = 0;
-    while ((int64_t(1) << bits) <= G) ++bits;  // keys in [0, G]
-    return (bits + kMaxDigitBits - 1) / kMaxDigitBits;
-}
-
-static int sort_bits(int64_t G)
-{
-    int bits = 0;
-    while ((int64_t(1) << bits) <= G) ++bits;
-    return bits;
-}
-
-void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int64_t n, int gx,
-                 int gy, int gz, const DomainRec* dom, SortBuffers& b, hipStream_t st)
-{
-    const int nblk = int((n + kSortTile - 1) / kSortTile);
-    const int bits = sort_bits(int64_t(gx) * gy * gz);
-    const int passes = (bits + kMaxDigitBits - 1) / kMaxDigitBits;
+    static_assert(kThreads * ITEMS * (2048 >> WIDTH) >= kSortTileItems, "counts buffer");
+    constexpr int kTile = kThreads * ITEMS;
+    const int nblk = int((n + kTile - 1) / kTile);
+    const int passes = (bits + WIDTH - 1) / WIDTH;
     const int width = (bits + passes - 1) / passes;
     const int nb = 1 << width;
+    const dim3 grid(round8(nblk)), block(kThreads);
     const int32_t* kin = b.keys0;
     const int32_t* vin = nullptr;
     int32_t* kout[2] = {b.keysA, b.keysB};
@@ -1732,24 +1761,47 @@ void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int6
     for (int p = 0; p < passes; ++p) {
         const int shift = width * p;
         if (p == 0)
-            hipLaunchKernelGGL(k_radix_count<true>, dim3(round8(nblk)), dim3(kThreads), 0, st,
-                               parts, stride, masks, gx, gy, gz, b.keys0, n, shift, width,
-                               b.counts, nblk, dom);
+            hipLaunchKernelGGL((k_radix_count<true, ITEMS, WIDTH>), grid, block, 0, st, parts,
+                               stride, masks, gx, gy, gz, b.keys0, n, shift, width, b.counts, nblk,
+                               dom);
         else
-            hipLaunchKernelGGL(k_radix_count<false>, dim3(round8(nblk)), dim3(kThreads), 0, st,
+            hipLaunchKernelGGL((k_radix_count<false, ITEMS, WIDTH>), grid, block, 0, st,
                                (const double*)nullptr, int64_t(0), (const uint8_t*)nullptr, gx,
                                gy, gz, const_cast<int32_t*>(kin), n, shift, width, b.counts,
                                nblk, dom);
-        hipLaunchKernelGGL(k_radix_scan, dim3(nb), dim3(kThreads), 0, st, b.counts, nblk,
-                           b.totals, dom);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(round8(nblk)), dim3(kThreads), 0, st, kin, vin,
-                           n, shift, width, b.counts, b.totals, nblk, kout[p & 1], vout[p & 1],
-                           dom);
+        hipLaunchKernelGGL(k_radix_scan, dim3(nb), block, 0, st, b.counts, nblk, b.totals, dom);
+        hipLaunchKernelGGL((k_radix_scatter<ITEMS, WIDTH>), grid, block, 0, st, kin, vin, n, shift,
+                           width, b.counts, b.totals, nblk, kout[p & 1], vout[p & 1], dom);
         kin = kout[p & 1];
         vin = vout[p & 1];
     }
-    b.sorted_keys = const_cast<int32_t*>(kin);
     b.perm = const_cast<int32_t*>(vin);
+}
+
+void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int64_t n, int gx,
+                 int gy, int gz, const DomainRec* dom, SortBuffers& b, hipStream_t st)
+{
+    const int64_t G = int64_t(gx) * gy * gz;
+    int bits = 0;
+    while ((int64_t(1) << bits) <= G) ++bits;  // keys in [0, G]
+    auto go = [&](auto f) { f(parts, stride, masks, n, gx, gy, gz, dom, b, bits, st); };
+    // Tile: small enough to fill the chip, large enough for the scan of the
+    // tiles' counts.  Whole sort with tiles of 1024 / 2048 / 4096 items, us:
+    // 1e5 particles 37 / 47 / 69, 1e6 56 / 62 / 80, 2e6 79 / 80 / 94, 4e6 125 /
+    // 116 / 120, 1.6e7 589 / 430 / 395 (4096 and one load per round before: 98
+    // at 1e5, 123 at 2e6).  Digits of 9 bits where they take fewer passes, with
+    // the small tiles: 1e5 particles on 32x32x64, 2 passes 30, 3 passes 37; of
+    // 10 bits they gain nothing (2e6 on 64x64x64: 85 against 80).
+    if (n <= 2500000) {
+        if ((bits + kWideDigitBits - 1) / kWideDigitBits < (bits + kMaxDigitBits - 1) / kMaxDigitBits)
+            go(launch_sort_tiles<4, kWideDigitBits>);
+        else
+            go(launch_sort_tiles<4, kMaxDigitBits>);
+    } else if (n <= 8000000) {
+        go(launch_sort_tiles<8, kMaxDigitBits>);
+    } else {
+        go(launch_sort_tiles<16, kMaxDigitBits>);
+    }
 }
 
 void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, const int32_t* perm,
