@@ -284,7 +284,8 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
     }
     const int32_t* dep_perm = nullptr;
     if (do_sort) {
-        launch_sort(b->parts, b->stride, b->masks, n, g.gx, g.gy, g.gz, c->dom, c->sb, st);
+        launch_sort(b->parts, b->stride, b->masks, n, g.gx, g.gy, g.gz, c->dom, c->sb,
+                    local_dep ? nullptr : c->scratch, st);
         c->sorted_n = n;
         if (do_reorder)
             launch_reorder(b->parts, b->stride, b->masks, n, c->sb.perm, c->scratch, c->smask,
@@ -293,16 +294,17 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
     }
     ev[2] = mark(c, st);
     // after a reorder the cell-sorted bunch is the gathered copy until the
-    // kick writes it back
+    // kick writes it back; a deposit through the permutation reads the sort's
+    // packed particles there
     c->reordering = do_reorder;
-    const double* dp = do_reorder ? c->scratch : b->parts;
+    const double* dp = do_reorder || dep_perm ? c->scratch : b->parts;
     const int64_t ds = do_reorder ? n : b->stride;
     const uint8_t* dm = do_reorder ? c->smask : b->masks;
     if (!c->fp32) {
-        launch_deposit<double>(dp, ds, dm, dep_perm, local_dep, n, g.gx, g.gy, g.gz, c->dom,
+        launch_deposit<double>(dp, ds, dm, dep_perm, n, g.gx, g.gy, g.gz, c->dom,
                                static_cast<double*>(c->rho), st);
     } else {
-        launch_deposit<float>(dp, ds, dm, dep_perm, local_dep, n, g.gx, g.gy, g.gz, c->dom,
+        launch_deposit<float>(dp, ds, dm, dep_perm, n, g.gx, g.gy, g.gz, c->dom,
                               static_cast<float*>(c->rho), st);
     }
     ev[3] = mark(c, st);

@@ -56,8 +56,11 @@ void launch_step_begin(StepCtl* ctl, hipStream_t st);
 // scheduled maps before the kick (the first step's first half-step)
 void launch_maps_sched(double* parts, int64_t stride, const uint8_t* masks, int64_t n,
                        const Sched& sc, hipStream_t st);
+// packed non-null: the key pass also leaves the particles there as (x, y, z,
+// active) records of 4 doubles, 32-byte aligned, in storage order.
 void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int64_t n, int gx,
-                 int gy, int gz, const DomainRec* dom, SortBuffers& b, hipStream_t st);
+                 int gy, int gz, const DomainRec* dom, SortBuffers& b, double* packed,
+                 hipStream_t st);
 void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, const int32_t* perm,
                     double* scratch, uint8_t* smask, const DomainRec* dom, hipStream_t st);
 // Deposit (k_deposit_tile) of windows through an LDS node tile of each
@@ -66,12 +69,12 @@ void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, co
 // weights; then k_rho_peak records the density peak in the domain record.
 template <typename R>
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
-                    const int32_t* perm, bool local, int64_t n, int gx, int gy, int gz,
-                    DomainRec* dom, R* rho, hipStream_t st);
+                    const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom, R* rho,
+                    hipStream_t st);
 template <>
 void launch_deposit<float>(const double* parts, int64_t stride, const uint8_t* masks,
-                           const int32_t* perm, bool local, int64_t n, int gx, int gy, int gz,
-                           DomainRec* dom, float* rho, hipStream_t st);
+                           const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
+                           float* rho, hipStream_t st);
 template <typename R>
 void launch_efield(const R* phi, int gx, int gy, int gz, const DomainRec* dom,
                    typename vec4<R>::type* E, hipStream_t st);

@@ -499,6 +499,13 @@ __device__ __forceinline__ unsigned part_block()
     return blockIdx.x;
 }
 
+// A particle for the deposit through a permutation, which reads in random
+// order: one 32-byte read instead of one line in each of three columns and the
+// masks.  Written by the key pass.
+struct alignas(32) Packed {
+    double x, y, z, active;
+};
+
 // The per-tile digit counts: entry (digit d, tile b), digit-major (the scan
 // reads a digit's row contiguously; measured faster than tile-major rows,
 // whose column reads in the scan cost more than the count pass's scattered
@@ -597,7 +604,8 @@ template <bool KEYS, int ITEMS, int WIDTH>
 __global__ __launch_bounds__(kThreads) void k_radix_count(
     const double* __restrict__ parts, int64_t stride, const uint8_t* __restrict__ masks, int gx,
     int gy, int gz, int32_t* __restrict__ keys, int64_t n, int shift, int width,
-    int32_t* __restrict__ counts, int nblk, const DomainRec* __restrict__ dom)
+    int32_t* __restrict__ counts, int nblk, const DomainRec* __restrict__ dom,
+    Packed* __restrict__ packed)
 {
     constexpr int kWaves = kThreads / 64;
     constexpr int kTile = kThreads * ITEMS;
@@ -635,7 +643,10 @@ __global__ __launch_bounds__(kThreads) void k_radix_count(
                 const int64_t i = base + (r0 + j) * 64 + lane;
                 const int32_t key = cell_key(m[j] != 0, x[j], y[j], z[j], gx, gy, gz, d);
                 kk[r0 + j] = i < n ? key : -1;
-                if (i < n) keys[i] = key;
+                if (i < n) {
+                    keys[i] = key;
+                    if (packed) packed[i] = Packed{x[j], y[j], z[j], m[j] ? 1.0 : 0.0};
+                }
             }
         }
     } else {
@@ -1064,13 +1075,21 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     } else {
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
-            int64_t j = min(base + q, n - 1);
-            if (PERM) j = perm[j];
-            x[q] = parts[j];
-            y[q] = parts[j + 2 * stride];
-            z[q] = parts[j + 4 * stride];
-            const uint8_t mask = masks[j];
-            m[q] = base + q < n ? mask : uint8_t(0);
+            const int64_t j = min(base + q, n - 1);
+            uint8_t active;
+            if (PERM) {
+                const Packed p = reinterpret_cast<const Packed*>(parts)[perm[j]];
+                x[q] = p.x;
+                y[q] = p.y;
+                z[q] = p.z;
+                active = p.active != 0.0;
+            } else {
+                x[q] = parts[j];
+                y[q] = parts[j + 2 * stride];
+                z[q] = parts[j + 4 * stride];
+                active = masks[j];
+            }
+            m[q] = base + q < n ? active : uint8_t(0);
         }
     }
     int ix[PER], iy[PER], iz[PER];
@@ -1772,7 +1791,7 @@ void launch_step_begin(StepCtl* ctl, hipStream_t st)
 template <int ITEMS, int WIDTH>
 static void launch_sort_tiles(const double* parts, int64_t stride, const uint8_t* masks, int64_t n,
                               int gx, int gy, int gz, const DomainRec* dom, SortBuffers& b,
-                              int bits, hipStream_t st)
+                              int bits, Packed* packed, hipStream_t st)
 {
     static_assert(kThreads * ITEMS * (2048 >> WIDTH) >= kSortTileItems, "counts buffer");
     constexpr int kTile = kThreads * ITEMS;
@@ -1790,12 +1809,12 @@ static void launch_sort_tiles(const double* parts, int64_t stride, const uint8_t
         if (p == 0)
             hipLaunchKernelGGL((k_radix_count<true, ITEMS, WIDTH>), grid, block, 0, st, parts,
                                stride, masks, gx, gy, gz, b.keys0, n, shift, width, b.counts, nblk,
-                               dom);
+                               dom, packed);
         else
             hipLaunchKernelGGL((k_radix_count<false, ITEMS, WIDTH>), grid, block, 0, st,
                                (const double*)nullptr, int64_t(0), (const uint8_t*)nullptr, gx,
                                gy, gz, const_cast<int32_t*>(kin), n, shift, width, b.counts,
-                               nblk, dom);
+                               nblk, dom, (Packed*)nullptr);
         hipLaunchKernelGGL(k_radix_scan, dim3(nb), block, 0, st, b.counts, nblk, b.totals, dom);
         hipLaunchKernelGGL((k_radix_scatter<ITEMS, WIDTH>), grid, block, 0, st, kin, vin, n, shift,
                            width, b.counts, b.totals, nblk, kout[p & 1], vout[p & 1], dom);
@@ -1806,12 +1825,13 @@ static void launch_sort_tiles(const double* parts, int64_t stride, const uint8_t
 }
 
 void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int64_t n, int gx,
-                 int gy, int gz, const DomainRec* dom, SortBuffers& b, hipStream_t st)
+                 int gy, int gz, const DomainRec* dom, SortBuffers& b, double* packed,
+                 hipStream_t st)
 {
     const int64_t G = int64_t(gx) * gy * gz;
     int bits = 0;
     while ((int64_t(1) << bits) <= G) ++bits;  // keys in [0, G]
-    auto go = [&](auto f) { f(parts, stride, masks, n, gx, gy, gz, dom, b, bits, st); };
+    auto go = [&](auto f) { f(parts, stride, masks, n, gx, gy, gz, dom, b, bits, reinterpret_cast<Packed*>(packed), st); };
     // Tile: small enough to fill the chip, large enough for the scan of the
     // tiles' counts.  Whole sort with tiles of 1024 / 2048 / 4096 items, us:
     // 1e5 particles 37 / 47 / 69, 1e6 56 / 62 / 80, 2e6 79 / 80 / 94, 4e6 125 /
@@ -1844,7 +1864,7 @@ void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, co
                        perm, n, scratch, smask, dom);
 }
 
-template <typename R, bool PERM>
+template <typename R>
 static void launch_deposit_tiles(const double* parts, int64_t stride, const uint8_t* masks,
                                  const int32_t* perm, int64_t n, int gx, int gy, int gz,
                                  DomainRec* dom, R* rho, hipStream_t st)
@@ -1860,8 +1880,10 @@ static void launch_deposit_tiles(const double* parts, int64_t stride, const uint
     // / 11.6 on 32x32x64; 4e5 on 64x64x128 14.8 / 12.6 / 15.5; 1e6 23.4 / 20.6 /
     // 19.9); one through a permutation, whose random reads want the wavefronts
     // (2e6 122 / 125 / 127, 4e6 266 / 273 / 279).
-    if (PERM || n < 250000)
-        launch(k_deposit_tile<R, 1, PERM>, 1);
+    if (perm != nullptr)
+        launch(k_deposit_tile<R, 1, true>, 1);
+    else if (n < 250000)
+        launch(k_deposit_tile<R, 1, false>, 1);
     else if (n < 750000)
         launch(k_deposit_tile<R, 2, false>, 2);
     else
@@ -1870,24 +1892,18 @@ static void launch_deposit_tiles(const double* parts, int64_t stride, const uint
 
 template <typename R>
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
-                    const int32_t* perm, bool local, int64_t n, int gx, int gy, int gz,
-                    DomainRec* dom, R* rho, hipStream_t st)
+                    const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom, R* rho,
+                    hipStream_t st)
 {
-    if (local)
-        launch_deposit_tiles<R, false>(parts, stride, masks, nullptr, n, gx, gy, gz, dom, rho, st);
-    else
-        launch_deposit_tiles<R, true>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
+    launch_deposit_tiles<R>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
 }
 
 template <>
 void launch_deposit<float>(const double* parts, int64_t stride, const uint8_t* masks,
-                           const int32_t* perm, bool local, int64_t n, int gx, int gy, int gz,
-                           DomainRec* dom, float* rho, hipStream_t st)
+                           const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
+                           float* rho, hipStream_t st)
 {
-    if (local)
-        launch_deposit_tiles<float, false>(parts, stride, masks, nullptr, n, gx, gy, gz, dom, rho, st);
-    else
-        launch_deposit_tiles<float, true>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
+    launch_deposit_tiles<float>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
     const int64_t G = int64_t(gx) * gy * gz;
     hipLaunchKernelGGL(k_rho_peak, dim3(grid_for(G / 8, 512)), dim3(kThreads), 0, st, rho, G, dom);
 }
@@ -1938,7 +1954,7 @@ void launch_populate(double* parts, int64_t stride, int64_t n, uint8_t* masks,
 }
 
 template void launch_deposit<double>(const double*, int64_t, const uint8_t*, const int32_t*,
-                                     bool, int64_t, int, int, int, DomainRec*, double*,
+                                     int64_t, int, int, int, DomainRec*, double*,
                                      hipStream_t);
 template void launch_efield<double>(const double*, int, int, int, const DomainRec*, double4*,
                                     hipStream_t);
