@@ -272,6 +272,9 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
         n > 0 && local_dep &&
         (sc.ctl != nullptr ? sc.sort_now != 0 : (c->applies % o.sort_period) == 0);
     const bool do_sort = n > 0 && (do_reorder || !local_dep);
+    // the first reorder meets the storage as it was populated or loaded
+    const bool records =
+        do_reorder && sc.ctl == nullptr && c->applies == 0 && n >= kRecordReorder;
     ev[0] = mark(c, st, true);
     launch_domain(b->parts, b->stride, b->masks, n, c->P, a, c->dom, sc, c->rho, c->rho_bytes,
                   st);
@@ -287,7 +290,10 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
         launch_sort(b->parts, b->stride, b->masks, n, g.gx, g.gy, g.gz, c->dom, c->sb,
                     local_dep ? nullptr : c->scratch, st);
         c->sorted_n = n;
-        if (do_reorder)
+        if (records)
+            launch_reorder_records(b->parts, b->stride, b->masks, n, c->sb.perm, c->scratch,
+                                   c->smask, c->dom, st);
+        else if (do_reorder)
             launch_reorder(b->parts, b->stride, b->masks, n, c->sb.perm, c->scratch, c->smask,
                            c->dom, st);
         if (!local_dep) dep_perm = c->sb.perm;
@@ -296,10 +302,10 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
     // after a reorder the cell-sorted bunch is the gathered copy until the
     // kick writes it back; a deposit through the permutation reads the sort's
     // packed particles there
-    c->reordering = do_reorder;
-    const double* dp = do_reorder || dep_perm ? c->scratch : b->parts;
-    const int64_t ds = do_reorder ? n : b->stride;
-    const uint8_t* dm = do_reorder ? c->smask : b->masks;
+    c->reordering = do_reorder && !records;
+    const double* dp = c->reordering || dep_perm ? c->scratch : b->parts;
+    const int64_t ds = c->reordering ? n : b->stride;
+    const uint8_t* dm = c->reordering ? c->smask : b->masks;
     if (!c->fp32) {
         launch_deposit<double>(dp, ds, dm, dep_perm, n, g.gx, g.gy, g.gz, c->dom,
                                static_cast<double*>(c->rho), st);

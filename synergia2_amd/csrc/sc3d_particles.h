@@ -63,6 +63,13 @@ void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int6
                  hipStream_t st);
 void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, const int32_t* perm,
                     double* scratch, uint8_t* smask, const DomainRec* dom, hipStream_t st);
+// Reorder in place, for a storage in unknown order; scratch and smask are used.
+// From kRecordReorder particles on (below, the bunch stays in the caches: 1e5
+// particles 11.6 us against 7.8).
+constexpr int64_t kRecordReorder = 250000;
+void launch_reorder_records(double* parts, int64_t stride, uint8_t* masks, int64_t n,
+                            const int32_t* perm, double* scratch, uint8_t* smask,
+                            const DomainRec* dom, hipStream_t st);
 // Deposit (k_deposit_tile) of windows through an LDS node tile of each
 // window's cell box; local: windows of the bunch storage (cell-sorted at every
 // reorder), else of the permutation `perm` of this step's sort.  FP32: unit

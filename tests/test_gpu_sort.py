@@ -1,4 +1,5 @@
-"""The cell sort's tiles (1024, 2048 or 4096 items by the particle count) and
+"""The first reorder (particle records from 250000 particles on) and the cell
+sort's tiles (1024, 2048 or 4096 items by the particle count) and
 digit widths (up to 8 bits, 9 where that saves a pass) at their edges: the
 permutation is the stable order of the keys, the keys the oracle's."""
 import numpy as np
@@ -7,7 +8,7 @@ import pytest
 import oracle as O
 import synergia2_amd as sc
 from helpers import BETA, gaussian_parts
-from test_gpu_parity import gpu_run, make_opts, oracle_kw, oracle_run
+from test_gpu_parity import check_kicked, gpu_run, make_opts, oracle_kw, oracle_run
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +33,23 @@ def test_sort_permutation(gpu, shape, n):
         rc, out = oracle_run(oracle_kw(shape), parts, masks, 1e10, dt, want=("keys",))
         assert rc == 0, O.last_error()
         assert np.array_equal(keys, out["keys"])
+
+
+@pytest.mark.parametrize("n", [249_999, 250_000, 250_003])
+def test_first_reorder(gpu, n):
+    shape = (24, 20, 32)
+    parts = gaussian_parts(n, (2e-3, 1e-4, 1.5e-3, 1e-4, 5e-3, 1e-4), seed=n)
+    masks = (np.arange(n) % 7).astype(np.uint8)  # 0 inactive, any other byte active
+    dt = 0.1 / (BETA * sc.C_LIGHT)
+    print(f"case first reorder {n}", flush=True)
+    rc, out = oracle_run(oracle_kw(shape), parts, (masks != 0).astype(np.uint8), 1e10, dt,
+                         want=("perm",))
+    assert rc == 0, O.last_error()
+    op, b = gpu_run(make_opts(shape, sort_period=1), parts, masks, 1e10, dt)
+    perm = op.debug(sc.DBG_PERM, n)
+    assert np.array_equal(perm, out["perm"])
+    got, gmasks = b.host()
+    assert np.array_equal(gmasks, masks[perm])
+    for c in (0, 2, 4, 6):
+        assert np.array_equal(got[c], parts[c][perm])
+    check_kicked(got, gmasks, out["parts"], parts)
