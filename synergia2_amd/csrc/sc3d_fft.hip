@@ -60,10 +60,18 @@ template <int L> struct Lines {
 // These launches are latency-bound and at 64x64x128 held two to four blocks
 // per CU.  Measured (us per kernel): at 64x64x128 FP64, x R2C 6.9 -> 5.8,
 // x C2R 5.6 -> 4.9, the two Green's column passes 17.5 -> 16.3; at
-// 128x128x256 FP32, the field x pass 50.4 -> 43.3.  k_green_x keeps Lines
-// (its FP32 pass at 128x128x256: Green's phase 112 -> 119 us with half).
+// 128x128x256 FP32, the field x pass 50.4 -> 43.3.  k_green_x has its
+// own count.
 template <int L> struct HalfLines {
     static constexpr int value = (512 / L) > 4 ? (512 / L) : 4;
+};
+// k_green_x: a thread evaluates ceil(NL (M + 1) / kThreads) points, so few
+// lines give the small grids more blocks and threads fewer rounds of a long
+// serial function, and 7 lines waste less of the last round than 8 (32x32x64
+// FP64, 32 -> 7 lines: 68 -> 307 blocks, 7.7 -> 4.6 us; 64x64x128, 16 -> 7:
+// FP64 13.2 -> 11.8, FP32 11.6 -> 10.2; 128x128x256 FP32, 8 -> 7: 45.3 -> 46.5).
+template <int M> struct GreenXLines {
+    static constexpr int value = M == 8 ? 28 : M == 16 ? 15 : M <= 64 ? 7 : 8;
 };
 // The solve's x R2C / C2R passes: half only for rows shorter than 128 (the
 // grids with few rows; at 128x128x256 the R2C pass is 18.5 us with Lines,
@@ -838,7 +846,7 @@ __global__ __launch_bounds__(kThreads) void k_green_x(
     const typename cplx<T>::type* __restrict__ tw2M, int gy, int gz, int green_fn)
 {
     using T2 = typename cplx<T>::type;
-    constexpr int NL = Lines<M>::value;
+    constexpr int NL = GreenXLines<M>::value;
     constexpr int Dx = 2 * M;
     __shared__ T2 buf[NL * LdsLine<M>::stride];
     __shared__ T2 twl[M];
@@ -972,7 +980,7 @@ template <typename T> struct Green {
                         const T2* tw, hipStream_t st)
         {
             int rows = (g.gz + 1) * (g.gy + 1);
-            hipLaunchKernelGGL((k_green_x<T, M>), dim3(nblocks(rows, Lines<M>::value), nj),
+            hipLaunchKernelGGL((k_green_x<T, M>), dim3(nblocks(rows, GreenXLines<M>::value), nj),
                                dim3(kThreads), 0, st, jobs, tw + twiddle_offset(M),
                                tw + twiddle_offset(2 * M), g.gy, g.gz, green_fn);
         }
