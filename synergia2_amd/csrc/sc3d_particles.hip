@@ -1398,11 +1398,15 @@ __global__ __launch_bounds__(kThreads, 4) void k_kick(double* __restrict__ parts
     const int64_t rs = COPY ? n : stride;
     const int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x;
     if (i >= n) return;
+    // the mask and all six coordinates in flight together (fused kick of the
+    // tracked cell, 4e6 particles: 180.9 -> 178.5 us)
     const uint8_t on = COPY ? smasks[i] : masks[i];
-    if (!COPY && !on) return;
-    // all six coordinates are loaded up front (independent loads in flight)
     double x = rd[i], y = rd[i + 2 * rs], cdt = rd[i + 4 * rs];
     double xp = rd[i + rs], yp = rd[i + 3 * rs], dpop = rd[i + 5 * rs];
+    if (!COPY) {
+        asm volatile("" ::"v"(x), "v"(y), "v"(cdt), "v"(xp), "v"(yp), "v"(dpop));
+        if (!on) return;
+    }
     double ox, oy, oz;
     int ix, iy, iz;
     bool in = grid_cell(x, lx, ihx, gx, ix, ox);
@@ -1451,7 +1455,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_kick(double* __restrict__ parts
     parts[i + 5 * stride] = dpop;
 }
 
-// The kick without maps over windows of the bunch storage (kKickPer
+// The kick without maps over windows of the bunch storage (PER
 // particles per lane, lane-interleaved so every load is coalesced) with the
 // field of each window's box of nodes staged in LDS: the storage is
 // cell-sorted at every reorder, so a window's particles share few nodes, and
@@ -1469,10 +1473,11 @@ __global__ __launch_bounds__(kThreads, 4) void k_kick(double* __restrict__ parts
 // multiply-adds in the interpolation and the cheaper cell test (391 -> 310
 // VALU instructions per particle): 61.0 -> 58.5 / 247 -> 233 us per launch,
 // 73 bytes per particle at 5.0 TB/s; k_kick with one drift fused 75.7 -> 69.7.
-constexpr int kKickPer = 2;
+// All of a lane's loads in flight together, no branch between them: 58.3 ->
+// 54.2 / 234.6 -> 226.8 us.
 constexpr int kKickNodes = 1024;
 
-template <typename R, bool COPY>
+template <typename R, bool COPY, int PER>
 __global__ __launch_bounds__(kThreads) void k_kick_tile(
     double* __restrict__ parts, int64_t stride, uint8_t* __restrict__ masks, int64_t n, int gx,
     int gy, int gz, const DomainRec* __restrict__ dom, const typename vec4<R>::type* __restrict__ E,
@@ -1486,44 +1491,46 @@ __global__ __launch_bounds__(kThreads) void k_kick_tile(
     const double ihx = dom->inv_h[0], ihy = dom->inv_h[1], ihz = dom->inv_h[2];
     const double factor = kick_factor<R>(*dom);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int64_t base = int64_t(blockIdx.x) * (kThreads * kKickPer) + t;
+    const int64_t base = int64_t(blockIdx.x) * (kThreads * PER) + t;
     const double* __restrict__ rd = COPY ? src : parts;
     const int64_t rs = COPY ? n : stride;
-    double x[kKickPer], y[kKickPer], cdt[kKickPer], xp[kKickPer], yp[kKickPer], dpop[kKickPer];
-    double ox[kKickPer], oy[kKickPer], oz[kKickPer];
-    int ix[kKickPer], iy[kKickPer], iz[kKickPer];
-    bool act[kKickPer], in[kKickPer];
+    double x[PER], y[PER], cdt[PER], xp[PER], yp[PER], dpop[PER];
+    double ox[PER], oy[PER], oz[PER];
+    int ix[PER], iy[PER], iz[PER];
+    double id[PER];  // COPY only
+    uint8_t on[PER];
+    bool in[PER];
     int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {-1, -1, -1};
+    // every load in flight together; a lane past n reads the last particle
 #pragma unroll
-    for (int q = 0; q < kKickPer; ++q) {
+    for (int q = 0; q < PER; ++q) {
+        const int64_t i = min(base + int64_t(q) * kThreads, n - 1);
+        on[q] = COPY ? smasks[i] : masks[i];
+        x[q] = rd[i];
+        y[q] = rd[i + 2 * rs];
+        cdt[q] = rd[i + 4 * rs];
+        xp[q] = rd[i + rs];
+        yp[q] = rd[i + 3 * rs];
+        dpop[q] = rd[i + 5 * rs];
+        if (COPY) id[q] = rd[i + 6 * rs];
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
         const int64_t i = base + int64_t(q) * kThreads;
-        act[q] = false;
-        x[q] = y[q] = cdt[q] = xp[q] = yp[q] = dpop[q] = 0.0;
-        if (i < n) {
-            const uint8_t on = COPY ? smasks[i] : masks[i];
-            act[q] = on != 0;
-            x[q] = rd[i];
-            y[q] = rd[i + 2 * rs];
-            cdt[q] = rd[i + 4 * rs];
-            xp[q] = rd[i + rs];
-            yp[q] = rd[i + 3 * rs];
-            dpop[q] = rd[i + 5 * rs];
-            if (COPY) {
-                masks[i] = on;
-                parts[i] = x[q];
-                parts[i + 2 * stride] = y[q];
-                parts[i + 4 * stride] = cdt[q];
-                parts[i + 6 * stride] = rd[i + 6 * rs];
-            }
+        if (COPY && i < n) {
+            masks[i] = on[q];
+            parts[i] = x[q];
+            parts[i + 2 * stride] = y[q];
+            parts[i + 4 * stride] = cdt[q];
+            parts[i + 6 * stride] = id[q];
         }
-        in[q] = grid_cell(x[q], lx, ihx, gx, ix[q], ox[q]);
-        in[q] = grid_cell(y[q], ly, ihy, gy, iy[q], oy[q]) && in[q];
-        in[q] = grid_cell(cdt[q], lz, ihz, gz, iz[q], oz[q]) && in[q] && act[q];
-        if (in[q]) {
-            lo[0] = min(lo[0], ix[q]); hi[0] = max(hi[0], ix[q]);
-            lo[1] = min(lo[1], iy[q]); hi[1] = max(hi[1], iy[q]);
-            lo[2] = min(lo[2], iz[q]); hi[2] = max(hi[2], iz[q]);
-        }
+        const bool in_x = grid_cell(x[q], lx, ihx, gx, ix[q], ox[q]);
+        const bool in_y = grid_cell(y[q], ly, ihy, gy, iy[q], oy[q]);
+        const bool in_z = grid_cell(cdt[q], lz, ihz, gz, iz[q], oz[q]);
+        in[q] = in_x & in_y & in_z & (on[q] != 0) & (i < n);
+        lo[0] = min(lo[0], in[q] ? ix[q] : INT32_MAX); hi[0] = max(hi[0], in[q] ? ix[q] : -1);
+        lo[1] = min(lo[1], in[q] ? iy[q] : INT32_MAX); hi[1] = max(hi[1], in[q] ? iy[q] : -1);
+        lo[2] = min(lo[2], in[q] ? iz[q] : INT32_MAX); hi[2] = max(hi[2], in[q] ? iz[q] : -1);
     }
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -1565,7 +1572,7 @@ __global__ __launch_bounds__(kThreads) void k_kick_tile(
         __syncthreads();
     }
 #pragma unroll
-    for (int q = 0; q < kKickPer; ++q) {
+    for (int q = 0; q < PER; ++q) {
         if (COPY ? base + int64_t(q) * kThreads >= n : !in[q]) continue;
         if (in[q]) {
             R ex[8], ey[8], ez[8];
@@ -1980,14 +1987,19 @@ void launch_kick(double* parts, int64_t stride, uint8_t* masks, int64_t n, int g
     if (n <= 0) return;
     const bool copy = src != nullptr;
     if (prog.n == 0 && !sc.progs) {
-        constexpr int win = kThreads * kKickPer;
-        const dim3 grid(unsigned((n + win - 1) / win));
-        if (copy)
-            hipLaunchKernelGGL((k_kick_tile<R, true>), grid, dim3(kThreads), 0, st, parts, stride,
-                               masks, n, gx, gy, gz, dom, E, pref, 1.0 / pref, m, src, smasks);
+        auto tiles = [&](auto kernel, int64_t win) {
+            hipLaunchKernelGGL(kernel, dim3(unsigned((n + win - 1) / win)), dim3(kThreads), 0, st,
+                               parts, stride, masks, n, gx, gy, gz, dom, E, pref, 1.0 / pref, m,
+                               src, smasks);
+        };
+        // one particle per lane where two would leave CUs idle (kick us, 1 / 2
+        // per lane: 1e4 particles 5.6 / 6.1, 1e6 20.4 / 20.8, 4e6 60.0 / 54.2)
+        if (n < 1000000)
+            copy ? tiles(k_kick_tile<R, true, 1>, kThreads)
+                 : tiles(k_kick_tile<R, false, 1>, kThreads);
         else
-            hipLaunchKernelGGL((k_kick_tile<R, false>), grid, dim3(kThreads), 0, st, parts,
-                               stride, masks, n, gx, gy, gz, dom, E, pref, 1.0 / pref, m, src, smasks);
+            copy ? tiles(k_kick_tile<R, true, 2>, 2 * kThreads)
+                 : tiles(k_kick_tile<R, false, 2>, 2 * kThreads);
         return;
     }
     const dim3 grid(unsigned((n + kThreads - 1) / kThreads));

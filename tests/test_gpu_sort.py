@@ -1,4 +1,5 @@
-"""The first reorder (particle records from 250000 particles on) and the cell
+"""The first reorder (particle records from 250000 particles on) with the kick
+that follows (two particles per lane from 1e6 on), and the cell
 sort's tiles (1024, 2048 or 4096 items by the particle count) and
 digit widths (up to 8 bits, 9 where that saves a pass) at their edges: the
 permutation is the stable order of the keys, the keys the oracle's."""
@@ -35,7 +36,7 @@ def test_sort_permutation(gpu, shape, n):
         assert np.array_equal(keys, out["keys"])
 
 
-@pytest.mark.parametrize("n", [249_999, 250_000, 250_003])
+@pytest.mark.parametrize("n", [249_999, 250_000, 250_003, 999_999, 1_000_003])
 def test_first_reorder(gpu, n):
     shape = (24, 20, 32)
     parts = gaussian_parts(n, (2e-3, 1e-4, 1.5e-3, 1e-4, 5e-3, 1e-4), seed=n)
