@@ -205,6 +205,27 @@ __device__ __forceinline__ int xcd_group()
 #endif
 }
 
+// The passes below issue a block's loads before they look at the domain
+// record's error mark: one memory latency instead of two (kernels of a few
+// microseconds wait for little else).  No predicate stands before a load
+// either: a line past the end loads the last one and is not stored.  With
+// global instead of flat accesses (in_memory) and 32-bit lane offsets, us:
+// 128x128x256 FP32 z field 87.8 -> 82.7, y 52 -> 46, x 43.6 -> 30.7, Green's
+// columns 27.6 -> 19.6 and 21.2 -> 15.1 (each stored value loaded once);
+// 64x64x128 FP32 y 13.8 -> 11.6, x 9.1 -> 7.1; 32x32x64 FP64, all eight passes
+// 37.8 -> 33.0.
+__device__ __forceinline__ void loads_issued() { asm volatile("" ::: "memory"); }
+
+// Element at a wavefront-uniform address plus a lane's 32-bit byte offset (the
+// workspaces of these lengths stay below 4 GiB): one address register for
+// all of a lane's elements instead of two each.
+template <typename T>
+__device__ __forceinline__ T& lane_at(T* uniform, uint32_t bytes)
+{
+    using C = std::conditional_t<std::is_const_v<T>, const char, char>;
+    return *reinterpret_cast<T*>(reinterpret_cast<C*>(uniform) + bytes);
+}
+
 // ---------------------------------------------------------------------------
 // x pass, forward: real rows of the rho octant -> half spectrum rows of S.
 // rows r in [0, gz*gy); input row r is rho + r*gx (gx = M reals); the
@@ -222,33 +243,41 @@ __global__ __launch_bounds__(kThreads) void k_x_r2c(const GridJob* __restrict__ 
     __shared__ T2 buf[NL * LdsLine<M>::stride];
     __shared__ T2 twl[M];
     const GridJob& J = jobs[blockIdx.y];
-    const R* __restrict__ rho = static_cast<const R*>(J.rho);
-    T2* __restrict__ S = static_cast<T2*>(J.S);
-    const DomainRec* dom = J.dom;
-    if (dom->error) return;
+    const R* __restrict__ rho = in_memory(static_cast<const R*>(J.rho));
+    T2* __restrict__ S = in_memory(static_cast<T2*>(J.S));
+    const DomainRec* dom = in_memory(J.dom);
+    const int error = dom->error;
     const int r0 = blockIdx.x * NL;
     const int Hx = M + 1;
     // precision form: the unit-weight density is scaled to unit peak here,
     // before any transform arithmetic (the peak returns at the kick)
     const float peak = __int_as_float(dom->rho_peak);
     const bool unit_peak = sizeof(R) == sizeof(float) && peak > 0.0f;
-    // load: NL consecutive rows are NL*M contiguous reals = NL*M/2 complex
+    // load: NL consecutive rows are NL*M contiguous reals = NL*M/2 complex,
+    // the lower halves of the lines
+    constexpr int K = NL * M / 2 / kThreads;
+    static_assert(K * kThreads == NL * M / 2, "whole rounds");
     const T2* src = reinterpret_cast<const T2*>(rho + int64_t(r0) * M);
-    for (int e = threadIdx.x; e < NL * M; e += kThreads) {
-        int line = e / M, n = e % M;
-        T2 v;
-        if (n < M / 2 && r0 + line < nrows) {
-            v = src[line * (M / 2) + n];
-            if (unit_peak) {
-                v.x = R(v.x / peak);
-                v.y = R(v.y / peak);
-            }
-        } else {
-            v.x = R(0); v.y = R(0);
-        }
-        buf[LdsLine<M>::at(line, n)] = v;
-    }
+    const int last = (nrows - r0) * (M / 2) - 1;
+    T2 in[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) in[i] = src[min(int(threadIdx.x) + i * kThreads, last)];
     load_twiddles<T2, M>(twl, twM);
+    loads_issued();
+    if (error) return;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int e = threadIdx.x + i * kThreads;
+        const int line = e / (M / 2), n = e % (M / 2);
+        T2 v = in[i], zero;
+        if (unit_peak) {
+            v.x = R(v.x / peak);
+            v.y = R(v.y / peak);
+        }
+        zero.x = R(0); zero.y = R(0);
+        buf[LdsLine<M>::at(line, n)] = v;
+        buf[LdsLine<M>::at(line, n + M / 2)] = zero;
+    }
     __syncthreads();
     lds_fft<T2, M, NL, false>(buf, twl);
     // post-process: X[k] = 1/2 (A + (-i) w^k B), A = Z[k] + conj Z[M-k],
@@ -288,34 +317,41 @@ __global__ __launch_bounds__(kThreads) void k_x_c2r(const GridJob* __restrict__ 
     __shared__ T2 buf[NL * LdsLine<M>::stride];
     __shared__ T2 twl[M];
     const GridJob& J = jobs[blockIdx.y];
-    const T2* __restrict__ S = static_cast<const T2*>(J.S);
-    R* __restrict__ phi = static_cast<R*>(J.phi);
-    const DomainRec* dom = J.dom;
-    if (dom->error) return;
+    const T2* __restrict__ S = in_memory(static_cast<const T2*>(J.S));
+    R* __restrict__ phi = in_memory(static_cast<R*>(J.phi));
+    const DomainRec* dom = in_memory(J.dom);
+    const int error = dom->error;
     const int r0 = blockIdx.x * NL;
     const int Hx = M + 1;
-    for (int e = threadIdx.x; e < NL * M; e += kThreads) {
-        int line = e / M, k = e % M;
-        int r = r0 + line;
-        T2 v;
-        if (r < nrows) {
-            int z = r / gy, y = r - z * gy;
-            const T2* row = S + (int64_t(z) * Dy + y) * Hx;
-            T2 xk = row[k];
-            T2 xm = row[M - k];
-            if (k == 0) { xk.y = R(0); xm.y = R(0); }
-            T2 A, B;
-            A.x = xk.x + xm.x; A.y = xk.y - xm.y;
-            B.x = xk.x - xm.x; B.y = xk.y + xm.y;
-            T2 Cc = cmul_conj(B, tw2M[k]);  // conj(w^k) * B
-            v.x = A.x - Cc.y;
-            v.y = A.y + Cc.x;
-        } else {
-            v.x = R(0); v.y = R(0);
-        }
-        buf[LdsLine<M>::at(line, k)] = v;
+    constexpr int K = NL * M / kThreads;
+    static_assert(K * kThreads == NL * M, "whole rounds");
+    T2 xk[K], xm[K], w[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int e = threadIdx.x + i * kThreads;
+        const int k = e % M, r = min(r0 + e / M, nrows - 1);
+        const int z = r / gy, y = r - z * gy;
+        const T2* row = S + (int64_t(z) * Dy + y) * Hx;
+        xk[i] = row[k];
+        xm[i] = row[M - k];
+        w[i] = tw2M[k];
     }
     load_twiddles<T2, M>(twl, twM);
+    loads_issued();
+    if (error) return;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int e = threadIdx.x + i * kThreads;
+        const int line = e / M, k = e % M;
+        if (k == 0) { xk[i].y = R(0); xm[i].y = R(0); }
+        T2 A, B, v;
+        A.x = xk[i].x + xm[i].x; A.y = xk[i].y - xm[i].y;
+        B.x = xk[i].x - xm[i].x; B.y = xk[i].y + xm[i].y;
+        T2 Cc = cmul_conj(B, w[i]);  // conj(w^k) * B
+        v.x = A.x - Cc.y;
+        v.y = A.y + Cc.x;
+        buf[LdsLine<M>::at(line, k)] = v;
+    }
     __syncthreads();
     lds_fft<T2, M, NL, true>(buf, twl);
     T2* dst = reinterpret_cast<T2*>(phi + int64_t(r0) * M);
@@ -488,28 +524,26 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     __shared__ T2 buf[NL * L];
     __shared__ T2 twl[L];
     const GridJob& J = jobs[blockIdx.y];
-    T2* __restrict__ S_ = static_cast<T2*>(J.S);
-    const DomainRec* dom = J.dom;
-    if (dom->error) return;
+    T2* __restrict__ S_ = in_memory(static_cast<T2*>(J.S));
+    const DomainRec* dom = in_memory(J.dom);
+    const int error = dom->error;
     const int line = int(threadIdx.x) % NL, j = int(threadIdx.x) / NL;
     const int l = xcd_group() * NL + line;
     const bool live = l < nlines;
-    int64_t base = 0;
-    if (live) {
-        const int plane = l / lpp, c = l - plane * lpp;
-        base = plane * plane_stride + c;
-    }
+    const int lc = min(l, nlines - 1);
+    const int plane = lc / lpp;
+    const uint32_t at =
+        uint32_t((plane * plane_stride + (lc - plane * lpp) + j * pstride) * int64_t(sizeof(T2)));
     T2* lb = buf + line * L;
     const int sw = line & (RegSwz<L, T2>::G - 1);
-    for (int e = threadIdx.x; e < L; e += NL * TPL) twl[e] = tw[e];
     // MODE 2: the Green's values of the elements this thread multiplies (the
     // outputs of the last forward pass), fetched with the line's loads
     R gv[E];
     if constexpr (MODE == 2) {
-        const R* __restrict__ ghat = static_cast<const R*>(J.ghat);
+        const R* __restrict__ ghat = in_memory(static_cast<const R*>(J.ghat));
         constexpr int rl = S::radix(S::np - 1, false), Bl = L / rl, Ql = E / rl;
         const int Dy = lpp / Hx;
-        const int ky = l / Hx, kx = l - ky * Hx;
+        const int ky = lc / Hx, kx = lc - ky * Hx;
         const int my = ky <= Dy / 2 ? ky : Dy - ky;
 #pragma unroll
         for (int q = 0; q < Ql; ++q)
@@ -517,7 +551,7 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
             for (int s = 0; s < rl; ++s) {
                 const int p = j + q * TPL + s * Bl;
                 const int mz = p <= L / 2 ? p : L - p;
-                gv[q * rl + s] = live ? ghat[(int64_t(mz) * (gy + 1) + my) * Hx + kx] : R(0);
+                gv[q * rl + s] = lane_at(ghat, uint32_t((mz * (gy + 1) + my) * Hx + kx) * uint32_t(sizeof(R)));
             }
     }
     // inputs of the first pass: elements b + s * L / r, b = j + q * TPL; the
@@ -531,15 +565,17 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     for (int q = 0; q < Qf; ++q)
 #pragma unroll
         for (int s = 0; s < rf; ++s) {
-            const int p = j + q * TPL + s * Bf;
             const bool in = MODE == 1 || s < rf / 2;
-            if (in && live) {
-                v[q * rf + s] = S_[base + p * pstride];
+            if (in) {
+                v[q * rf + s] = lane_at(S_ + (q * TPL + s * Bf) * pstride, at);
             } else {
                 v[q * rf + s].x = R(0);
                 v[q * rf + s].y = R(0);
             }
         }
+    for (int e = threadIdx.x; e < L; e += NL * TPL) twl[e] = tw[e];
+    loads_issued();
+    if (error) return;
     reg_fft<T2, L, MODE == 1>(v, lb, j, sw, twl, false);
     if constexpr (MODE == 2) {
 #pragma unroll
@@ -559,8 +595,8 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     for (int q = 0; q < Ql; ++q)
 #pragma unroll
         for (int s = 0; s < rl; ++s) {
-            const int p = j + q * TPL + s * Bl;
-            if (MODE == 0 || s < rl / 2) S_[base + p * pstride] = v[q * rl + s];
+            if (MODE == 0 || s < rl / 2)
+                lane_at(S_ + (q * TPL + s * Bl) * pstride, at) = v[q * rl + s];
         }
 }
 
@@ -598,7 +634,8 @@ __device__ __forceinline__ T2 mul_minus_i(T2 v, R s)
 template <typename T2>
 __device__ __forceinline__ auto sin_2pi(const T2* __restrict__ tw, int k, int L)
 {
-    return (k == 0 || 2 * k == L) ? decltype(tw[0].y)(0) : -tw[k].y;
+    const auto y = tw[k].y;
+    return (k == 0 || 2 * k == L) ? decltype(tw[0].y)(0) : -y;
 }
 
 // The z' and y' passes register-resident (the register layout of the
@@ -619,22 +656,23 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     __shared__ T2 buf[NL * L];
     __shared__ T2 twl[L];
     const GridJob& J = jobs[blockIdx.y];
-    T2* __restrict__ S1 = static_cast<T2*>(J.S);
-    T2* __restrict__ S2 = static_cast<T2*>(J.S2);
-    const R* __restrict__ ghat = static_cast<const R*>(J.ghat);
-    const DomainRec* dom = J.dom;
-    if (dom->error) return;
+    T2* __restrict__ S1 = in_memory(static_cast<T2*>(J.S));
+    T2* __restrict__ S2 = in_memory(static_cast<T2*>(J.S2));
+    const R* __restrict__ ghat = in_memory(static_cast<const R*>(J.ghat));
+    const DomainRec* dom = in_memory(J.dom);
+    const int error = dom->error;
     const R ihz = R(dom->inv_h[2]);
     const int line = int(threadIdx.x) % NL, j = int(threadIdx.x) / NL;
     const int l = xcd_group() * NL + line;
     const bool live = l < nlines;
+    const int lc = min(l, nlines - 1);
+    const uint32_t at = uint32_t(j * nlines + lc) * uint32_t(sizeof(T2));
     T2* lb = buf + line * L;
     const int sw = line & (RegSwz<L, T2>::G - 1);
-    for (int e = threadIdx.x; e < L; e += NL * TPL) twl[e] = tw[e];
     // Green's values of the outputs of the last forward pass
     constexpr int rl = S::radix(S::np - 1, false), Bl = L / rl, Ql = E / rl;
     const int Dy = nlines / Hx;
-    const int ky = l / Hx, kx = l - ky * Hx;
+    const int ky = lc / Hx, kx = lc - ky * Hx;
     const int my = ky <= Dy / 2 ? ky : Dy - ky;
     R gv[E];
 #pragma unroll
@@ -643,19 +681,22 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
         for (int s = 0; s < rl; ++s) {
             const int p = j + q * TPL + s * Bl;
             const int mz = p <= L / 2 ? p : L - p;
-            gv[q * rl + s] = live ? ghat[(int64_t(mz) * (gy + 1) + my) * Hx + kx] : R(0);
+            gv[q * rl + s] = lane_at(ghat, uint32_t((mz * (gy + 1) + my) * Hx + kx) * uint32_t(sizeof(R)));
         }
     // z < gz = L/2 loaded: elements j + s * TPL, s < E/2
     T2 v[E];
 #pragma unroll
     for (int s = 0; s < E; ++s) {
-        if (s < E / 2 && live) {
-            v[s] = S1[int64_t(j + s * TPL) * nlines + l];
+        if (s < E / 2) {
+            v[s] = lane_at(S1 + int64_t(s * TPL) * nlines, at);
         } else {
             v[s].x = R(0);
             v[s].y = R(0);
         }
     }
+    for (int e = threadIdx.x; e < L; e += NL * TPL) twl[e] = tw[e];
+    loads_issued();
+    if (error) return;
     reg_fft<T2, L, false>(v, lb, j, sw, twl, false);
     T2 keep[E];
 #pragma unroll
@@ -667,7 +708,7 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     reg_fft<T2, L, true>(v, lb, j, sw, twl, true);
     if (live) {
 #pragma unroll
-        for (int s = 0; s < E / 2; ++s) S1[int64_t(j + s * TPL) * nlines + l] = v[s];
+        for (int s = 0; s < E / 2; ++s) lane_at(S1 + int64_t(s * TPL) * nlines, at) = v[s];
     }
 #pragma unroll
     for (int q = 0; q < Ql; ++q)
@@ -679,12 +720,12 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     reg_fft<T2, L, true>(v, lb, j, sw, twl, true);
     if (live) {
 #pragma unroll
-        for (int s = 0; s < E / 2; ++s) S2[int64_t(j + s * TPL) * nlines + l] = v[s];
+        for (int s = 0; s < E / 2; ++s) lane_at(S2 + int64_t(s * TPL) * nlines, at) = v[s];
     }
 }
 
 template <typename R, int L>
-__global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) void k_y_field_reg(
+__global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads), 4) void k_y_field_reg(
     const GridJob* __restrict__ jobs, const typename cplx<R>::type* __restrict__ tw, int nlines,
     int gy, int Hx)
 {
@@ -695,56 +736,61 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     __shared__ T2 buf[NL * L];
     __shared__ T2 twl[L];
     const GridJob& J = jobs[blockIdx.y];
-    T2* __restrict__ S1 = static_cast<T2*>(J.S);
-    T2* __restrict__ S2 = static_cast<T2*>(J.S2);
-    const DomainRec* dom = J.dom;
-    if (dom->error) return;
+    T2* __restrict__ S1 = in_memory(static_cast<T2*>(J.S));
+    T2* __restrict__ S2 = in_memory(static_cast<T2*>(J.S2));
+    const DomainRec* dom = in_memory(J.dom);
+    const int error = dom->error;
     const R ihy = R(dom->inv_h[1]);
     const int line = int(threadIdx.x) % NL, j = int(threadIdx.x) / NL;
     const int l = xcd_group() * NL + line;
     const bool live = l < nlines;
-    int64_t base = 0;
-    if (live) {
-        const int z = l / Hx, c = l - z * Hx;
-        base = int64_t(z) * L * Hx + c;  // L = Dy rows of Hx
-    }
+    const int lc = min(l, nlines - 1), z = lc / Hx;
+    // L = Dy rows of Hx
+    const uint32_t at = uint32_t((z * L + j) * Hx + (lc - z * Hx)) * uint32_t(sizeof(T2));
     T2* lb = buf + line * L;
     const int sw = line & (RegSwz<L, T2>::G - 1);
-    for (int e = threadIdx.x; e < L; e += NL * TPL) twl[e] = tw[e];
     // inputs of the first inverse pass (radix r0): elements b + s * L / r0
     constexpr int r0 = S::radix(0, true), B0 = L / r0, Q0 = E / r0;
     T2 a[E], b[E], c[E];
+    R sy[E];
 #pragma unroll
     for (int q = 0; q < Q0; ++q)
 #pragma unroll
         for (int s = 0; s < r0; ++s) {
             const int p = j + q * TPL + s * B0, e = q * r0 + s;
-            if (live) {
-                a[e] = S1[base + int64_t(p) * Hx];
-                c[e] = S2[base + int64_t(p) * Hx];
-            } else {
-                a[e].x = R(0); a[e].y = R(0);
-                c[e] = a[e];
-            }
-            b[e] = mul_minus_i(a[e], sin_2pi(tw, p, L) * ihy);
+            a[e] = lane_at(S1 + (q * TPL + s * B0) * Hx, at);
+            sy[e] = sin_2pi(tw, p, L);
         }
+    for (int e = threadIdx.x; e < L; e += NL * TPL) twl[e] = tw[e];
+    loads_issued();
+    if (error) return;
+#pragma unroll
+    for (int e = 0; e < E; ++e) b[e] = mul_minus_i(a[e], sy[e] * ihy);
     // rows y < gy kept: the inverse passes end with radix E, elements
     // j + s * TPL, s < E/2
     reg_fft<T2, L, true>(a, lb, j, sw, twl, false);
     if (live) {
 #pragma unroll
-        for (int s = 0; s < E / 2; ++s) S1[base + int64_t(j + s * TPL) * Hx] = a[s];
+        for (int s = 0; s < E / 2; ++s) lane_at(S1 + s * TPL * Hx, at) = a[s];
     }
+    // the S2 line, under the second transform: with the first line it would
+    // take the kernel past the 128 registers of two blocks per CU (its stores
+    // come after the barriers of its own transform)
+#pragma unroll
+    for (int q = 0; q < Q0; ++q)
+#pragma unroll
+        for (int s = 0; s < r0; ++s)
+            c[q * r0 + s] = lane_at(S2 + (q * TPL + s * B0) * Hx, at);
     reg_fft<T2, L, true>(b, lb, j, sw, twl, true);
     if (live) {
 #pragma unroll
         for (int s = 0; s < E / 2; ++s)
-            S1[base + int64_t(gy + j + s * TPL) * Hx] = b[s];
+            lane_at(S1 + (gy + s * TPL) * Hx, at) = b[s];
     }
     reg_fft<T2, L, true>(c, lb, j, sw, twl, true);
     if (live) {
 #pragma unroll
-        for (int s = 0; s < E / 2; ++s) S2[base + int64_t(j + s * TPL) * Hx] = c[s];
+        for (int s = 0; s < E / 2; ++s) lane_at(S2 + s * TPL * Hx, at) = c[s];
     }
 }
 
@@ -759,45 +805,60 @@ __global__ __launch_bounds__(kThreads) void k_x_field(
     __shared__ T2 buf[3 * NL * LdsLine<M>::stride];
     __shared__ T2 twl[M];
     const GridJob& J = jobs[blockIdx.y];
-    const T2* __restrict__ S = static_cast<const T2*>(J.S);
-    const T2* __restrict__ S2 = static_cast<const T2*>(J.S2);
-    T4* __restrict__ E = static_cast<T4*>(J.E);
-    const DomainRec* dom = J.dom;
-    if (dom->error) return;
+    const T2* __restrict__ S = in_memory(static_cast<const T2*>(J.S));
+    const T2* __restrict__ S2 = in_memory(static_cast<const T2*>(J.S2));
+    T4* __restrict__ E = in_memory(static_cast<T4*>(J.E));
+    const DomainRec* dom = in_memory(J.dom);
+    const int error = dom->error;
     const R ihx = R(dom->inv_h[0]);
     const int nrows = gz * gy;
     const int r0 = blockIdx.x * NL;
     const int Hx = M + 1;
-    for (int e = threadIdx.x; e < NL * M; e += kThreads) {
-        int line = e / M, k = e % M;
-        int r = r0 + line;
-        int z = r / gy, y = r - z * gy;
+    constexpr int K = NL * M / kThreads;
+    static_assert(K * kThreads == NL * M, "whole rounds");
+    T2 xk[K][3], xm[K][3], w[K];
+    R sk[K], sm[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int e = threadIdx.x + i * kThreads;
+        const int k = e % M, r = min(r0 + e / M, nrows - 1);
+        const int z = r / gy, y = r - z * gy;
+        const T2* row = S + (int64_t(z) * Dy + y) * Hx;
+        const T2* row2 = S2 + (int64_t(z) * Dy + y) * Hx;
+        xk[i][0] = row[k];
+        xm[i][0] = row[M - k];
+        xk[i][1] = row[int64_t(gy) * Hx + k];
+        xm[i][1] = row[int64_t(gy) * Hx + M - k];
+        xk[i][2] = row2[k];
+        xm[i][2] = row2[M - k];
+        w[i] = tw2M[k];
+        sk[i] = sin_2pi(tw2M, k, 2 * M);
+        sm[i] = sin_2pi(tw2M, M - k, 2 * M);
+    }
+    load_twiddles<T2, M>(twl, twM);
+    loads_issued();
+    if (error) return;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int e = threadIdx.x + i * kThreads;
+        const int line = e / M, k = e % M;
 #pragma unroll
         for (int f = 0; f < 3; ++f) {
-            T2 v;
-            if (r < nrows) {
-                const T2* row = f == 2 ? S2 + (int64_t(z) * Dy + y) * Hx
-                                       : S + (int64_t(z) * Dy + y + (f == 1 ? gy : 0)) * Hx;
-                T2 xk = row[k];
-                T2 xm = row[M - k];
-                if (k == 0) { xk.y = R(0); xm.y = R(0); }
-                if (f == 0) {  // x derivative, D_x(k) for k and M-k (2M = Dx)
-                    xk = mul_minus_i(xk, sin_2pi(tw2M, k, 2 * M) * ihx);
-                    xm = mul_minus_i(xm, sin_2pi(tw2M, M - k, 2 * M) * ihx);
-                }
-                T2 A, B;
-                A.x = xk.x + xm.x; A.y = xk.y - xm.y;
-                B.x = xk.x - xm.x; B.y = xk.y + xm.y;
-                T2 Cc = cmul_conj(B, tw2M[k]);
-                v.x = A.x - Cc.y;
-                v.y = A.y + Cc.x;
-            } else {
-                v.x = R(0); v.y = R(0);
+            T2 p = xk[i][f], m = xm[i][f];
+            if (k == 0) { p.y = R(0); m.y = R(0); }
+            if (f == 0) {  // x derivative, D_x(k) for k and M-k (2M = Dx)
+                p = mul_minus_i(p, sk[i] * ihx);
+                m = mul_minus_i(m, sm[i] * ihx);
             }
+            T2 A, B, v;
+            A.x = p.x + m.x; A.y = p.y - m.y;
+            B.x = p.x - m.x; B.y = p.y + m.y;
+            T2 Cc = cmul_conj(B, w[i]);
+            v.x = A.x - Cc.y;
+            v.y = A.y + Cc.x;
             buf[LdsLine<M>::at((f * NL + line), k)] = v;
         }
     }
-    load_twiddles<T2, M>(twl, twM);
     __syncthreads();
     lds_fft<T2, M, 3 * NL, true>(buf, twl);
     for (int e = threadIdx.x; e < NL * M; e += kThreads) {
@@ -833,9 +894,9 @@ __global__ __launch_bounds__(kThreads) void k_x_field(
 template <typename T> __device__ __forceinline__ T* green_buffer(const GridJob& J)
 {
     if constexpr (sizeof(T) == sizeof(double))
-        return J.ghat64;
+        return in_memory(J.ghat64);
     else
-        return static_cast<float*>(J.ghat);
+        return in_memory(static_cast<float*>(J.ghat));
 }
 
 // G1: rows (Z<=gz, Y<=gy) of the doubled grid: generate, R2C along x, keep
@@ -853,8 +914,8 @@ __global__ __launch_bounds__(kThreads) void k_green_x(
     __shared__ T row[NL * (M + 1)];
     const GridJob& J = jobs[blockIdx.y];
     T* __restrict__ ghat = green_buffer<T>(J);
-    const DomainRec* dom = J.dom;
-    if (dom->error || !dom->ghat_dirty) return;
+    const DomainRec* dom = in_memory(J.dom);
+    if (dom->error | (dom->ghat_dirty == 0)) return;  // one wait
     const int nrows = (gz + 1) * (gy + 1);
     const int r0 = blockIdx.x * NL;
     const double hx = dom->h[0], hy = dom->h[1], hz = dom->h[2];
@@ -918,33 +979,40 @@ __global__ __launch_bounds__(kThreads) void k_green_cols(
     __shared__ T2 twl[L];
     const GridJob& J = jobs[blockIdx.y];
     T* __restrict__ ghat = green_buffer<T>(J);
-    const DomainRec* dom = J.dom;
-    if (dom->error || !dom->ghat_dirty) return;
+    const DomainRec* dom = in_memory(J.dom);
+    if (dom->error | (dom->ghat_dirty == 0)) return;  // one wait
     const int l0 = xcd_group() * NL;
-    auto addr = [&](int c, int p) -> int64_t {
-        int plane = c / Hx, kx = c - plane * Hx;
-        if (AXIS == 1) return (int64_t(plane) * (gy + 1) + p) * Hx + kx;
-        return (int64_t(p) * (gy + 1) + plane) * Hx + kx;
-    };
     // element e: p = e / (2 NL), column q = e % (2 NL) of the block's 2 NL
-    // consecutive columns (runs of 2 NL doubles along kx)
-    for (int e = threadIdx.x; e < 2 * NL * L; e += kThreads) {
-        int p = e / (2 * NL), q = e % (2 * NL);
-        int c = 2 * l0 + q;
-        T v = c < ncols ? ghat[addr(c, p <= L / 2 ? p : L - p)] : T(0);
-        T2* slot = &buf[LdsLine<L>::at((q >> 1), p)];
-        if (q & 1) slot->y = v; else slot->x = v;
+    // consecutive columns (runs of 2 NL values along kx); a thread keeps its
+    // column.  Each stored value is loaded once, for p and L - p.
+    constexpr int W = 2 * NL, PT = kThreads / W, K = L / 2 / PT;
+    static_assert(PT * W == kThreads && K * PT == L / 2, "whole rounds");
+    const int q = threadIdx.x % W, p0 = threadIdx.x / W;
+    const int c = 2 * l0 + q, cc = min(c, ncols - 1);
+    const int plane = cc / Hx;
+    const int64_t at0 = AXIS == 1 ? int64_t(plane) * (gy + 1) * Hx + (cc - plane * Hx) : cc;
+    const int64_t ps = AXIS == 1 ? Hx : int64_t(gy + 1) * Hx;
+    T v[K], vm = T(0);
+#pragma unroll
+    for (int i = 0; i < K; ++i) v[i] = ghat[at0 + (p0 + i * PT) * ps];
+    if (p0 == 0) vm = ghat[at0 + L / 2 * ps];
+    auto put = [&](int p, T x) {
+        reinterpret_cast<T*>(&buf[LdsLine<L>::at((q >> 1), p)])[q & 1] = x;
+    };
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int p = p0 + i * PT;
+        put(p, v[i]);
+        if (p > 0) put(L - p, v[i]);
     }
+    if (p0 == 0) put(L / 2, vm);
     load_twiddles<T2, L>(twl, tw);
     __syncthreads();
     lds_fft<T2, L, NL, false>(buf, twl);
-    for (int e = threadIdx.x; e < 2 * NL * (L / 2 + 1); e += kThreads) {
-        int p = e / (2 * NL), q = e % (2 * NL);
-        int c = 2 * l0 + q;
-        if (c < ncols) {
-            const T2 z = buf[LdsLine<L>::at((q >> 1), p)];
-            ghat[addr(c, p)] = (q & 1) ? z.y : z.x;
-        }
+    if (c >= ncols) return;
+    for (int p = p0; p <= L / 2; p += PT) {
+        const T2 z = buf[LdsLine<L>::at((q >> 1), p)];
+        ghat[at0 + p * ps] = (q & 1) ? z.y : z.x;
     }
 }
 

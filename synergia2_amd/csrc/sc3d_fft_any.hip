@@ -695,9 +695,9 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_x_r2c(
 {
     using T2 = typename cplx<R>::type;
     const GridJob& J = jobs[blockIdx.y];
-    const R* __restrict__ in = FULL ? C : static_cast<const R*>(J.rho);
-    T2* __restrict__ S = FULL ? chat : static_cast<T2*>(J.S);
-    const DomainRec* dom = J.dom;
+    const R* __restrict__ in = FULL ? C : in_memory(static_cast<const R*>(J.rho));
+    T2* __restrict__ S = FULL ? chat : in_memory(static_cast<T2*>(J.S));
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error || (FULL && !dom->ghat_dirty)) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_row_lane(a);
@@ -747,9 +747,9 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_x_c2r(
 {
     using T2 = typename cplx<R>::type;
     const GridJob& J = jobs[blockIdx.y];
-    const T2* __restrict__ S = static_cast<const T2*>(J.S);
-    R* __restrict__ phi = static_cast<R*>(J.phi);
-    const DomainRec* dom = J.dom;
+    const T2* __restrict__ S = in_memory(static_cast<const T2*>(J.S));
+    R* __restrict__ phi = in_memory(static_cast<R*>(J.phi));
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_row_lane(a);
@@ -798,8 +798,8 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_cols(
 {
     using T2 = typename cplx<R>::type;
     const GridJob& J = jobs[blockIdx.y];
-    T2* __restrict__ S = MODE == 3 ? over : static_cast<T2*>(J.S);
-    const DomainRec* dom = J.dom;
+    T2* __restrict__ S = MODE == 3 ? over : in_memory(static_cast<T2*>(J.S));
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error || (MODE == 3 && !dom->ghat_dirty)) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_lane(a);
@@ -816,8 +816,8 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_cols(
     if constexpr (MODE == 2) {
         const int Dy = lpp / Hx;
         const int ky = l / Hx, kx = l - ky * Hx;
-        const R* ghat = static_cast<const R*>(J.ghat);
-        const T2* chat = static_cast<const T2*>(J.chat);
+        const R* ghat = in_memory(static_cast<const R*>(J.ghat));
+        const T2* chat = in_memory(static_cast<const T2*>(J.chat));
         const AnySpectrum<T2, R> sp{ghat + min(ky, Dy - ky) * Hx + kx, chat ? chat + l : nullptr,
                                     (gy + 1) * Hx, lpp, L, m.twl, R(0)};
         any_convolve<1>(a, q, m.buf, m.alt, m.twl, io, sp);
@@ -840,9 +840,9 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_z_field(
 {
     using T2 = typename cplx<R>::type;
     const GridJob& J = jobs[blockIdx.y];
-    const R* __restrict__ ghat = static_cast<const R*>(J.ghat);
-    const T2* __restrict__ chat = static_cast<const T2*>(J.chat);
-    const DomainRec* dom = J.dom;
+    const R* __restrict__ ghat = in_memory(static_cast<const R*>(J.ghat));
+    const T2* __restrict__ chat = in_memory(static_cast<const T2*>(J.chat));
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_lane(a);
@@ -852,8 +852,8 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_z_field(
     const bool live = q.line >= 0 && l < nlines;
     if (!live) l = 0;
     const int ky = l / Hx, kx = l - ky * Hx;
-    const AnyColumn<T2, true, true> io{static_cast<T2*>(second ? J.S2 : J.S) + l, nlines, L / 2,
-                                       live};
+    const AnyColumn<T2, true, true> io{in_memory(static_cast<T2*>(second ? J.S2 : J.S)) + l, nlines,
+                                       L / 2, live};
     const AnySpectrum<T2, R> sp{ghat + min(ky, Dy - ky) * Hx + kx, chat ? chat + l : nullptr,
                                 (gy + 1) * Hx, nlines, L, m.twl, R(dom->inv_h[2])};
     any_convolve<2>(a, q, m.buf, m.alt, m.twl, io, sp);
@@ -887,7 +887,7 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_y_field(
 {
     using T2 = typename cplx<R>::type;
     const GridJob& J = jobs[blockIdx.y];
-    const DomainRec* dom = J.dom;
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_lane(a);
@@ -898,7 +898,7 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_y_field(
     if (!live) l = 0;
     const int z = l / Hx;
     AnyFieldColumn<T2, R> io;
-    T2* in = static_cast<T2*>(f == 2 ? J.S2 : J.S) + int64_t(z) * L * Hx + (l - z * Hx);
+    T2* in = in_memory(static_cast<T2*>(f == 2 ? J.S2 : J.S)) + int64_t(z) * L * Hx + (l - z * Hx);
     io.col = in + (f == 1 ? gy * Hx : 0);
     io.ps = Hx;
     io.half = gy;
@@ -922,10 +922,10 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_x_field(
     using T2 = typename cplx<R>::type;
     using T4 = typename vec4_of<R>::type;
     const GridJob& J = jobs[blockIdx.y];
-    const T2* __restrict__ S = static_cast<const T2*>(J.S);
-    const T2* __restrict__ S2 = static_cast<const T2*>(J.S2);
-    T4* __restrict__ E = static_cast<T4*>(J.E);
-    const DomainRec* dom = J.dom;
+    const T2* __restrict__ S = in_memory(static_cast<const T2*>(J.S));
+    const T2* __restrict__ S2 = in_memory(static_cast<const T2*>(J.S2));
+    T4* __restrict__ E = in_memory(static_cast<T4*>(J.E));
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_row_lane(a);
@@ -993,7 +993,8 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_x_field(
 // ---------------------------------------------------------------------------
 template <typename T> __device__ __forceinline__ T* any_ghat(const GridJob& J)
 {
-    return sizeof(T) == sizeof(double) ? reinterpret_cast<T*>(J.ghat64) : static_cast<T*>(J.ghat);
+    return in_memory(sizeof(T) == sizeof(double) ? reinterpret_cast<T*>(J.ghat64)
+                                                 : static_cast<T*>(J.ghat));
 }
 
 template <typename T>
@@ -1004,7 +1005,7 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_green_x(
     using T2 = typename cplx<T>::type;
     const GridJob& J = jobs[blockIdx.y];
     T* __restrict__ ghat = any_ghat<T>(J);
-    const DomainRec* dom = J.dom;
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error || !dom->ghat_dirty) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_row_lane(a);
@@ -1073,7 +1074,7 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_green_cols(
     using T2 = typename cplx<T>::type;
     const GridJob& J = jobs[blockIdx.y];
     T* __restrict__ ghat = any_ghat<T>(J);
-    const DomainRec* dom = J.dom;
+    const DomainRec* dom = in_memory(J.dom);
     if (dom->error || !dom->ghat_dirty) return;
     AnyLds<T2> m = any_lds(a, tw);
     const AnyLane q = any_lane(a);

@@ -86,6 +86,15 @@ struct GridJob {
     void* chat;
 };
 
+// A pointer read from a job record, known to lie in device memory (the
+// compiler cannot know, and would use flat accesses, which also take the LDS
+// path and wait on its counter).
+template <typename T>
+__device__ __forceinline__ T* in_memory(T* p)
+{
+    return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+
 // Green's spectrum (when the job's cell size changed), transformed in R
 // (values evaluated in FP64).  All launches on `st`, asynchronous.
 template <typename R>
