@@ -71,8 +71,8 @@ typedef struct sc3d_options {
     int32_t precision;           /* SC3D_PRECISION_*; default FP64           */
     int32_t sort_period;         /* every N applies the particles are sorted
                                     by cell and the bunch storage is reordered
-                                    into that order (the deposit sorts windows
-                                    of the storage on the device in between);
+                                    into that order (the deposit works on
+                                    windows of the storage in between);
                                     0 = never reorder: sort on every apply and
                                     deposit through the permutation; default 24*/
 } sc3d_options;

@@ -146,7 +146,7 @@ struct MapProgram {
 // drift_unit's two correctly rounded square roots and its division cost about
 // 78 VALU instructions per drift and thin kick, most of them scaling and
 // special-case handling.  Here one reciprocal-square-root seed serves all
-// three (46 instructions), and the results are the same bits:
+// three (38 instructions), and the results are the same bits:
 //   y  ~ 1/sqrt(a), a = dp^2 - x'^2 - y'^2: hardware seed, one third-order
 //      step, about 1 ulp;
 //   s  = sqrt(a) from y (sc3d_exact.h);
@@ -161,7 +161,7 @@ struct MapProgram {
 // where one residual step cannot decide the rounding; there the path length
 // has a square root of its own).
 // Measured (4e6 particles, mean over the 10 steps of an O-F-O-D cell, 6
-// quadrupole slices among them): maps pass 266 -> 178 us, kick with maps fused
+// quadrupole slices among them): maps pass 266 -> 172 us, kick with maps fused
 // (whole step) 449 -> 364 us; a step of drifts alone stays at 54 us, its
 // 89 bytes per particle at 6.6 TB/s.  Four wavefronts per SIMD (<= 128 VGPRs,
 // no spills) need one particle per thread: the grid-stride loop's pointers
