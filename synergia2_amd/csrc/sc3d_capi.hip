@@ -28,12 +28,11 @@ thread_local std::string g_err;
 // context that simply reallocates on its next apply.
 void drop_particle_buffers(sc3d_ctx* c)
 {
+    dfree(c, c->sb.keys0);  // the first of the set
     for (void** p : {(void**)&c->sb.keys0, (void**)&c->sb.keysA, (void**)&c->sb.keysB,
                      (void**)&c->sb.valsA, (void**)&c->sb.valsB, (void**)&c->sb.counts,
-                     (void**)&c->sb.totals, (void**)&c->scratch, (void**)&c->smask}) {
-        dfree(c, *p);
+                     (void**)&c->sb.totals, (void**)&c->scratch, (void**)&c->smask})
         *p = nullptr;
-    }
     c->sb.perm = nullptr;
     c->pcap = 0;
     c->sorted_n = -1;
@@ -45,19 +44,17 @@ int ensure_particle_buffers(sc3d_ctx* c, int64_t n)
     drop_particle_buffers(c);
     const int64_t cap = n + n / 8 + 4096;
     const int64_t tiles = (cap + kSortTileItems - 1) / kSortTileItems;
-    int rc = dmalloc(c, &c->sb.keys0, cap);
-    if (!rc) rc = dmalloc(c, &c->sb.keysA, cap);
-    if (!rc) rc = dmalloc(c, &c->sb.keysB, cap);
-    if (!rc) rc = dmalloc(c, &c->sb.valsA, cap);
-    if (!rc) rc = dmalloc(c, &c->sb.valsB, cap);
-    if (!rc) rc = dmalloc(c, &c->sb.counts, 2048 * tiles);
-    if (!rc) rc = dmalloc(c, &c->sb.totals, 2048);
-    if (!rc) rc = dmalloc(c, &c->scratch, 7 * cap);
-    if (!rc) rc = dmalloc(c, &c->smask, cap);
-    if (rc) {
-        drop_particle_buffers(c);
-        return rc;
-    }
+    BufferSet set;
+    set.add(&c->sb.keys0, cap);
+    set.add(&c->sb.keysA, cap);
+    set.add(&c->sb.keysB, cap);
+    set.add(&c->sb.valsA, cap);
+    set.add(&c->sb.valsB, cap);
+    set.add(&c->sb.counts, 2048 * tiles);
+    set.add(&c->sb.totals, 2048);
+    set.add(&c->scratch, 7 * cap);
+    set.add(&c->smask, cap);
+    if (int rc = set.allocate(c)) return rc;
     c->pcap = cap;
     return 0;
 }
@@ -430,42 +427,42 @@ int sc3d_create(const sc3d_options* opt, sc3d_ctx** out)
     if (hipGetDevice(&c->device) != hipSuccess)
         return cleanup(fail(SC3D_ERR_HIP, "sc3d_create: no HIP device"));
     const int64_t rs = c->fp32 ? 4 : 8;
-    int rc = 0;
-    rc |= dmalloc(c, &c->dom, 1);
-    char* p = nullptr;
     c->rho_bytes = (g.G * rs + 15) / 16 * 16;
-    rc |= dmalloc(c, &p, c->rho_bytes);
-    c->rho = p;
-    rc |= dmalloc(c, &p, g.S_elems * 2 * rs);
-    c->S = p;
-    if (c->fp32) {
-        rc |= dmalloc(c, &p, g.S_elems * 2 * rs);
-        c->S2 = p;
-    } else {
-        rc |= dmalloc(c, &p, g.G * rs);
-        c->phi = p;
-    }
-    rc |= dmalloc(c, &p, g.G * 4 * rs);
-    c->E = p;
+    char *rho = nullptr, *S = nullptr, *S2 = nullptr, *phi = nullptr, *E = nullptr;
+    char *Cbuf = nullptr, *chat = nullptr;
+    BufferSet set;
+    set.add(&c->dom, 1);
+    set.add(&rho, c->rho_bytes);
+    set.add(&S, g.S_elems * 2 * rs);
     if (c->fp32)
-        rc |= dmalloc(c, &c->ghat32, g.Ghat_elems);
+        set.add(&S2, g.S_elems * 2 * rs);
     else
-        rc |= dmalloc(c, &c->ghat64, g.Ghat_elems);
-    rc |= dmalloc(c, &c->tw64, g.tw_elems);
-    rc |= dmalloc(c, &c->tw32, g.tw_elems);
-    rc |= dmalloc(c, &c->d_gj, 1);
+        set.add(&phi, g.G * rs);
+    set.add(&E, g.G * 4 * rs);
+    if (c->fp32)
+        set.add(&c->ghat32, g.Ghat_elems);
+    else
+        set.add(&c->ghat64, g.Ghat_elems);
+    set.add(&c->tw64, g.tw_elems);
+    set.add(&c->tw32, g.tw_elems);
+    set.add(&c->d_gj, 1);
     if (c->spectral_patch) {
-        rc |= dmalloc(c, &p, int64_t(g.Dz) * g.Dy * g.Dx * rs);
-        c->Cbuf = p;
-        rc |= dmalloc(c, &p, int64_t(g.Dz) * g.Dy * g.Hx * 2 * rs);
-        c->chat = p;
+        set.add(&Cbuf, int64_t(g.Dz) * g.Dy * g.Dx * rs);
+        set.add(&chat, int64_t(g.Dz) * g.Dy * g.Hx * 2 * rs);
     }
-    if (rc) return cleanup(rc);
+    if (c->npatch > 0) set.add(&c->d_patch, c->npatch);
+    if (int rc = set.allocate(c)) return cleanup(rc);
+    c->rho = rho;
+    c->S = S;
+    c->S2 = S2;
+    c->phi = phi;
+    c->E = E;
+    c->Cbuf = Cbuf;
+    c->chat = chat;
     if (c->spectral_patch &&
         hipMemset(c->Cbuf, 0, size_t(g.Dz) * g.Dy * g.Dx * rs) != hipSuccess)
         return cleanup(fail(SC3D_ERR_HIP, "sc3d_create: workspace initialisation failed"));
     if (c->npatch > 0) {
-        if (int rp = dmalloc(c, &c->d_patch, c->npatch)) return cleanup(rp);
         if (hipMemcpy(c->d_patch, patches.data(), patches.size() * sizeof(GreenPatch),
                       hipMemcpyHostToDevice) != hipSuccess)
             return cleanup(fail(SC3D_ERR_HIP, "sc3d_create: workspace initialisation failed"));

@@ -188,9 +188,7 @@ void release_graph(sc3d_server* s)
 void drop_job_buffers(Job* j)
 {
     if (j->ctx) sc3d_destroy(j->ctx);
-    for (void* p : {(void*)j->parts, (void*)j->masks, (void*)j->ctl, (void*)j->d_progs,
-                    (void*)j->d_dt})
-        if (p) (void)hipFree(p);
+    if (j->parts) (void)hipFree(j->parts);  // the others lie behind it
     j->ctx = nullptr;
     j->parts = nullptr;
     j->masks = nullptr;
@@ -205,11 +203,18 @@ int admit_alloc(sc3d_server* s, Job* j)
     const int64_t n = sp.n_particles;
     const sc3d_options o = job_options(sp, s->opt.precision, s->opt.sort_period);
     if (int rc = sc3d_create(&o, &j->ctx)) return rc;
-    HIP_TRY(hipMalloc(&j->parts, size_t(n) * 7 * sizeof(double)));
-    HIP_TRY(hipMalloc(&j->masks, size_t(n)));
-    HIP_TRY(hipMalloc(&j->ctl, sizeof(StepCtl)));
-    HIP_TRY(hipMalloc(&j->d_progs, j->progs.size() * sizeof(MapProgram)));
-    HIP_TRY(hipMalloc(&j->d_dt, j->dt.size() * sizeof(double)));
+    // one allocation for the job's own buffers, 256-byte aligned each
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t b_parts = up(size_t(n) * 7 * sizeof(double)), b_masks = up(size_t(n)),
+                 b_ctl = up(sizeof(StepCtl)), b_progs = up(j->progs.size() * sizeof(MapProgram)),
+                 b_dt = up(j->dt.size() * sizeof(double));
+    char* at = nullptr;
+    HIP_TRY(hipMalloc(&at, b_parts + b_masks + b_ctl + b_progs + b_dt));
+    j->parts = reinterpret_cast<double*>(at);
+    j->masks = reinterpret_cast<uint8_t*>(at += b_parts);
+    j->ctl = reinterpret_cast<StepCtl*>(at += b_masks);
+    j->d_progs = reinterpret_cast<MapProgram*>(at += b_ctl);
+    j->d_dt = reinterpret_cast<double*>(at += b_progs);
     StepCtl c{};
     c.turn_steps = sp.turn_steps;
     c.total_steps = sp.steps;
