@@ -273,7 +273,7 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
     const bool records =
         do_reorder && sc.ctl == nullptr && c->applies == 0 && n >= kRecordReorder;
     ev[0] = mark(c, st, true);
-    launch_domain(b->parts, b->stride, b->masks, n, c->P, a, c->dom, sc, c->rho, c->rho_bytes,
+    launch_domain(b->parts, b->stride, b->masks, n, c->P, a, c->dom, sc, c->sums, c->sums_bytes,
                   st);
     ev[1] = mark(c, st);
     if (green_st) {
@@ -303,13 +303,8 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
     const double* dp = c->reordering || dep_perm ? c->scratch : b->parts;
     const int64_t ds = c->reordering ? n : b->stride;
     const uint8_t* dm = c->reordering ? c->smask : b->masks;
-    if (!c->fp32) {
-        launch_deposit<double>(dp, ds, dm, dep_perm, n, g.gx, g.gy, g.gz, c->dom,
-                               static_cast<double*>(c->rho), st);
-    } else {
-        launch_deposit<float>(dp, ds, dm, dep_perm, n, g.gx, g.gy, g.gz, c->dom,
-                              static_cast<float*>(c->rho), st);
-    }
+    launch_deposit(dp, ds, dm, dep_perm, n, g.gx, g.gy, g.gz, c->dom, c->sums,
+                   c->fp32 ? static_cast<float*>(c->rho) : nullptr, st);
     ev[3] = mark(c, st);
     return SC3D_OK;
 }
@@ -427,12 +422,12 @@ int sc3d_create(const sc3d_options* opt, sc3d_ctx** out)
     if (hipGetDevice(&c->device) != hipSuccess)
         return cleanup(fail(SC3D_ERR_HIP, "sc3d_create: no HIP device"));
     const int64_t rs = c->fp32 ? 4 : 8;
-    c->rho_bytes = (g.G * rs + 15) / 16 * 16;
+    c->sums_bytes = (g.G * 8 + 15) / 16 * 16;
     char *rho = nullptr, *S = nullptr, *S2 = nullptr, *phi = nullptr, *E = nullptr;
     char *Cbuf = nullptr, *chat = nullptr;
     BufferSet set;
     set.add(&c->dom, 1);
-    set.add(&rho, c->rho_bytes);
+    set.add(&rho, (g.G * rs + 15) / 16 * 16);
     set.add(&S, g.S_elems * 2 * rs);
     if (c->fp32)
         set.add(&S2, g.S_elems * 2 * rs);
@@ -453,6 +448,8 @@ int sc3d_create(const sc3d_options* opt, sc3d_ctx** out)
     if (c->npatch > 0) set.add(&c->d_patch, c->npatch);
     if (int rc = set.allocate(c)) return cleanup(rc);
     c->rho = rho;
+    // precision form: the field is written after the density has been rounded
+    c->sums = reinterpret_cast<double*>(c->fp32 ? E : rho);
     c->S = S;
     c->S2 = S2;
     c->phi = phi;

@@ -19,7 +19,8 @@ struct sc3d_ctx {
     double* P = nullptr;
     int64_t P_cap = 0;
     void* rho = nullptr;
-    int64_t rho_bytes = 0;  // the density grid, rounded up to 16 bytes
+    double* sums = nullptr;  // FP64 density sums: rho, or (precision form) in E's buffer
+    int64_t sums_bytes = 0;  // rounded up to 16 bytes
     void* S = nullptr;
     void* S2 = nullptr;   // precision form: second spectrum workspace
     void* phi = nullptr;  // FP64 form only

@@ -72,16 +72,13 @@ void launch_reorder_records(double* parts, int64_t stride, uint8_t* masks, int64
                             const DomainRec* dom, hipStream_t st);
 // Deposit (k_deposit_tile) of windows through an LDS node tile of each
 // window's cell box; local: windows of the bunch storage (cell-sorted at every
-// reorder), else of the permutation `perm` of this step's sort.  FP32: unit
-// weights; then k_rho_peak records the density peak in the domain record.
-template <typename R>
+// reorder), else of the permutation `perm` of this step's sort.  sums: the
+// density, cleared (launch_domain).  rho32 non-null (precision form): unit
+// weights; k_rho_round then rounds the sums to rho32 and records the density
+// peak in the domain record.
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
-                    const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom, R* rho,
-                    hipStream_t st);
-template <>
-void launch_deposit<float>(const double* parts, int64_t stride, const uint8_t* masks,
-                           const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
-                           float* rho, hipStream_t st);
+                    const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
+                    double* sums, float* rho32, hipStream_t st);
 template <typename R>
 void launch_efield(const R* phi, int gx, int gy, int gz, const DomainRec* dom,
                    typename vec4<R>::type* E, hipStream_t st);

@@ -933,9 +933,11 @@ __global__ void k_fill(R* __restrict__ p, int64_t n, R v)
 // wavefront), the rest going to rho directly.  Those wide
 // windows lie at the two ends of the cell order (the tails of the bunch), so
 // the block order is rotated to start the last eighth of the windows
-// first and keep them off the end of the kernel.  The tile accumulates in
-// FP64 for both precisions (the precision form's unit weights are rounded
-// to FP32 once, at the global add).
+// first and keep them off the end of the kernel.  Tile and grid accumulate in
+// FP64 for both precisions; the precision form's unit-weight sums are rounded
+// once, by k_rho_round.  (Global adds in FP32 left each node an order-dependent
+// error of 6e-8; over a few steps that moved single particles across a cell
+// face, and so the slots of the next reorder, from one run to the next.)
 // Measured against the windowed kernel it replaces (LDS radix sort of each
 // window, lane runs, DPP segmented scan, LDS run list; PMC: 465 VALU
 // instructions per particle), deposit phase per step over sort periods of
@@ -1065,10 +1067,9 @@ __device__ __forceinline__ void tile_deposit(double* tile, int bx, int by, int b
 
 // The non-zero interior nodes of a tile (box at (bx, by, bz), nx x ny x ..,
 // `nodes` in all) into rho, node e of the thread's share first..step.
-template <typename R>
 __device__ __forceinline__ void tile_flush(const double* tile, int nodes, int first, int step,
                                            int bx, int by, int bz, int nx, int ny, int gx, int gy,
-                                           int gz, R* __restrict__ rho)
+                                           int gz, double* __restrict__ rho)
 {
     const uint32_t mx = small_magic(nx), my = small_magic(ny);
     for (int e = first; e < nodes; e += step) {
@@ -1077,7 +1078,7 @@ __device__ __forceinline__ void tile_flush(const double* tile, int nodes, int fi
         const int r = small_div(e, mx), rz = small_div(r, my);
         const int cx = bx + e - r * nx, cy = by + r - rz * ny, cz = bz + rz;
         if (cx > 0 && cx < gx - 1 && cy > 0 && cy < gy - 1 && cz > 0 && cz < gz - 1)
-            unsafeAtomicAdd(rho + (int64_t(cz) * gy + cy) * gx + cx, R(v));
+            unsafeAtomicAdd(rho + (int64_t(cz) * gy + cy) * gx + cx, v);
     }
 }
 
@@ -1094,11 +1095,13 @@ __device__ __forceinline__ void load_run(const double* __restrict__ p, double (&
     }
 }
 
-template <typename R, int PER, bool PERM>
+// UNIT (precision form): unit weights; w0 and the unit-peak scale return at
+// the kick.
+template <bool UNIT, int PER, bool PERM>
 __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     const double* __restrict__ parts, int64_t stride, const uint8_t* __restrict__ masks,
     const int32_t* __restrict__ perm, int64_t n, int gx, int gy, int gz,
-    const DomainRec* __restrict__ dom, R* __restrict__ rho)
+    const DomainRec* __restrict__ dom, double* __restrict__ rho)
 {
     __shared__ double tile[kTileNodes];
     __shared__ int box[kTileWaves][6];
@@ -1107,8 +1110,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     const LaneCorners lc(lane);
     const double lx = dom->left[0], ly = dom->left[1], lz = dom->left[2];
     const double ihx = dom->inv_h[0], ihy = dom->inv_h[1], ihz = dom->inv_h[2];
-    // precision form: unit weights (w0 and the unit-peak scale return at the kick)
-    const double w0 = sizeof(R) == sizeof(double) ? dom->w0 : 1.0;
+    const double w0 = UNIT ? 1.0 : dom->w0;
     // the last eighth of the windows (one tail of the bunch) first
     const int nb = int(gridDim.x), tail = nb / kTileTailDiv;
     const int blk = (int(blockIdx.x) + nb - tail) % nb;
@@ -1190,8 +1192,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
         __syncthreads();
         tile_deposit(tile, blo[0], blo[1], blo[2], nx, ny, lc, w0, ix, iy, iz, ok, ox, oy, oz);
         __syncthreads();
-        tile_flush<R>(tile, nodes, t, kTileThreads, blo[0], blo[1], blo[2], nx, ny, gx, gy, gz,
-                      rho);
+        tile_flush(tile, nodes, t, kTileThreads, blo[0], blo[1], blo[2], nx, ny, gx, gy, gz, rho);
         return;
     }
     // the window's box does not fit: this wavefront's own box in its quarter
@@ -1206,7 +1207,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
         tile_deposit(wtile, lo[0], lo[1], lo[2], wnx, wny, lc, w0, ix, iy, iz, ok, ox, oy, oz);
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        tile_flush<R>(wtile, wn, lane, 64, lo[0], lo[1], lo[2], wnx, wny, gx, gy, gz, rho);
+        tile_flush(wtile, wn, lane, 64, lo[0], lo[1], lo[2], wnx, wny, gx, gy, gz, rho);
         return;
     }
     // scattered particles (the sparse tails, or a storage out of cell order):
@@ -1239,25 +1240,25 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
             if (held == -1 || held == node)
                 unsafeAtomicAdd(&cval[slot], w[k]);
             else
-                unsafeAtomicAdd(rho + node, R(w[k]));
+                unsafeAtomicAdd(rho + node, w[k]);
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
     for (int e = lane; e < kCacheSlots; e += 64) {
         const int node = ckey[e];
-        if (node >= 0) unsafeAtomicAdd(rho + node, R(cval[e]));
+        if (node >= 0) unsafeAtomicAdd(rho + node, cval[e]);
     }
 }
 
-// Peak of the unit-weight FP32 density (all entries >= 0, so the IEEE bit
-// patterns order like the values): block max (wavefront butterflies, then
-// LDS), one integer atomicMax per block into the domain record (cleared by
-// k_domain_finish each apply); the grid is bounded so few atomics meet
-// (measured at 128x128x256: 8.9 us per launch over 512 blocks, 14.8 us with
-// 16-byte loads over 1024 blocks).
-__global__ __launch_bounds__(kThreads) void k_rho_peak(const float* __restrict__ rho, int64_t G,
-                                                       DomainRec* __restrict__ dom)
+// The precision form's density: the FP64 sums of unit weights rounded to FP32,
+// and the peak of that (all entries >= 0, so the IEEE bit patterns order like
+// the values): block max (wavefront butterflies, then LDS), one integer
+// atomicMax per block into the domain record (cleared by k_domain_finish each
+// apply); the grid is bounded so few atomics meet.
+__global__ __launch_bounds__(kThreads) void k_rho_round(const double* __restrict__ sums,
+                                                        float* __restrict__ rho, int64_t G,
+                                                        DomainRec* __restrict__ dom)
 {
     __shared__ float wmax[kThreads / 64];
     if (dom->error) return;
@@ -1266,13 +1267,21 @@ __global__ __launch_bounds__(kThreads) void k_rho_peak(const float* __restrict__
     const int64_t T = int64_t(gridDim.x) * kThreads;
     int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x;
     for (; i + 7 * T < G; i += 8 * T) {
-        float v[8];
+        double v[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = rho[i + u * T];
+        for (int u = 0; u < 8; ++u) v[u] = sums[i + u * T];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) m = fmaxf(m, v[u]);
+        for (int u = 0; u < 8; ++u) {
+            const float r = float(v[u]);
+            rho[i + u * T] = r;
+            m = fmaxf(m, r);
+        }
     }
-    for (; i < G; i += T) m = fmaxf(m, rho[i]);
+    for (; i < G; i += T) {
+        const float r = float(sums[i]);
+        rho[i] = r;
+        m = fmaxf(m, r);
+    }
     m = __int_as_float(wave_max(__float_as_int(m)));  // m >= 0: the bits order like the values
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -1933,10 +1942,10 @@ void launch_reorder_records(double* parts, int64_t stride, uint8_t* masks, int64
                        parts, stride, masks, dom);
 }
 
-template <typename R>
+template <bool UNIT>
 static void launch_deposit_tiles(const double* parts, int64_t stride, const uint8_t* masks,
                                  const int32_t* perm, int64_t n, int gx, int gy, int gz,
-                                 DomainRec* dom, R* rho, hipStream_t st)
+                                 DomainRec* dom, double* rho, hipStream_t st)
 {
     auto launch = [&](auto kernel, int per) {
         const int64_t win = kTileThreads * int64_t(per), nb = (n + win - 1) / win;
@@ -1950,31 +1959,27 @@ static void launch_deposit_tiles(const double* parts, int64_t stride, const uint
     // 19.9); one through a permutation, whose random reads want the wavefronts
     // (2e6 122 / 125 / 127, 4e6 266 / 273 / 279).
     if (perm != nullptr)
-        launch(k_deposit_tile<R, 1, true>, 1);
+        launch(k_deposit_tile<UNIT, 1, true>, 1);
     else if (n < 250000)
-        launch(k_deposit_tile<R, 1, false>, 1);
+        launch(k_deposit_tile<UNIT, 1, false>, 1);
     else if (n < 750000)
-        launch(k_deposit_tile<R, 2, false>, 2);
+        launch(k_deposit_tile<UNIT, 2, false>, 2);
     else
-        launch(k_deposit_tile<R, 4, false>, 4);
+        launch(k_deposit_tile<UNIT, 4, false>, 4);
 }
 
-template <typename R>
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
-                    const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom, R* rho,
-                    hipStream_t st)
+                    const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
+                    double* sums, float* rho32, hipStream_t st)
 {
-    launch_deposit_tiles<R>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
-}
-
-template <>
-void launch_deposit<float>(const double* parts, int64_t stride, const uint8_t* masks,
-                           const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
-                           float* rho, hipStream_t st)
-{
-    launch_deposit_tiles<float>(parts, stride, masks, perm, n, gx, gy, gz, dom, rho, st);
+    if (!rho32) {
+        launch_deposit_tiles<false>(parts, stride, masks, perm, n, gx, gy, gz, dom, sums, st);
+        return;
+    }
+    launch_deposit_tiles<true>(parts, stride, masks, perm, n, gx, gy, gz, dom, sums, st);
     const int64_t G = int64_t(gx) * gy * gz;
-    hipLaunchKernelGGL(k_rho_peak, dim3(grid_for(G / 8, 512)), dim3(kThreads), 0, st, rho, G, dom);
+    hipLaunchKernelGGL(k_rho_round, dim3(grid_for(G / 8, 512)), dim3(kThreads), 0, st, sums, rho32,
+                       G, dom);
 }
 
 template <typename R>
@@ -2027,9 +2032,6 @@ void launch_populate(double* parts, int64_t stride, int64_t n, uint8_t* masks,
                        masks, a);
 }
 
-template void launch_deposit<double>(const double*, int64_t, const uint8_t*, const int32_t*,
-                                     int64_t, int, int, int, DomainRec*, double*,
-                                     hipStream_t);
 template void launch_efield<double>(const double*, int, int, int, const DomainRec*, double4*,
                                     hipStream_t);
 template void launch_efield<float>(const float*, int, int, int, const DomainRec*, float4*,
