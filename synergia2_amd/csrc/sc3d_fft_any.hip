@@ -1039,7 +1039,10 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_green_x(
     }
 }
 
-// Real-even columns as one line (FP64: two), elements p <= L/2 stored.
+// Real-even columns as one line (FP64: two), elements p <= L/2 stored.  A last
+// column without a partner goes with zeros: whatever stood in the partner's
+// place would enter the stored real part, and another block's column may be
+// overwritten while it is read.
 template <typename T2, typename T> struct AnyEvenColumns {
     T *g0, *g1;
     int ps, L;
@@ -1050,7 +1053,8 @@ template <typename T2, typename T> struct AnyEvenColumns {
         for (int r = 0; r < N; ++r) {
             const int p = b + r * NB, e = min(p, L - p) * ps;
             v[r].x = g0[e];
-            v[r].y = any_rows_per<T2>() == 2 ? g1[e] : T(0);
+            const T y = any_rows_per<T2>() == 2 ? g1[e] : T(0);
+            v[r].y = on1 ? y : T(0);
         }
     }
     __device__ __forceinline__ void store1(int p, T2 v) const
@@ -1085,7 +1089,7 @@ __global__ __launch_bounds__(kAnyThreads, 4) void ga_green_cols(
         const int plane = c / Hx, kx = c - plane * Hx;
         return ghat + int64_t(plane) * (AXIS == 1 ? (gy + 1) * Hx : Hx) + kx;
     };
-    const AnyEvenColumns<T2, T> io{column(on0 ? c0 : 0), column(on1 ? c1 : 0),
+    const AnyEvenColumns<T2, T> io{column(on0 ? c0 : 0), column(on1 ? c1 : on0 ? c0 : 0),
                                    AXIS == 1 ? Hx : (gy + 1) * Hx, a.pl.L, on0, on1};
     any_columns<false>(a, q, m.buf, m.alt, m.twl, io);
 }
