@@ -320,7 +320,7 @@ void enqueue_grid(sc3d_ctx* const* ctxs, int nj, const GridJob* table, hipStream
         enqueue_green(ctxs, nj, table, st);
     ev[4] = mark(c, st);
     if (!c->fp32) {
-        launch_solve<double>(g, table, nj, c->tw64, st);
+        launch_solve<double>(g, table, nj, c->served, c->tw64, st);
         ev[5] = mark(c, st);
         for (int j = 0; j < nj; ++j) {
             sc3d_ctx* cj = ctxs[j];
@@ -332,7 +332,7 @@ void enqueue_grid(sc3d_ctx* const* ctxs, int nj, const GridJob* table, hipStream
     } else {
         // the field comes straight out of the spectrum (no potential, no
         // separate difference pass): sc3d_force stays empty in this form
-        launch_solve_field<float>(g, table, nj, c->tw32, st);
+        launch_solve_field<float>(g, table, nj, c->served, c->tw32, st);
         for (int j = 0; j < nj; ++j) launch_green_patches(ctxs[j], st);
         ev[5] = mark(c, st);
         ev[6] = mark(c, st);

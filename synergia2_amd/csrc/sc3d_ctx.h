@@ -15,6 +15,7 @@ struct sc3d_ctx {
     sc3d::Geometry g;
     int device = 0;
     bool fp32 = false;
+    bool served = false;  // a server's job: its applies may be no-ops (StepCtl::done)
     sc3d::DomainRec* dom = nullptr;
     double* P = nullptr;
     int64_t P_cap = 0;

@@ -214,6 +214,10 @@ __device__ __forceinline__ int xcd_group()
 // columns 27.6 -> 19.6 and 21.2 -> 15.1 (each stored value loaded once);
 // 64x64x128 FP32 y 13.8 -> 11.6, x 9.1 -> 7.1; 32x32x64 FP64, all eight passes
 // 37.8 -> 33.0.
+// SERVED: a served job stays in the captured launches for some iterations after
+// its last step and must cost them nothing, so its blocks wait for the mark
+// first (an iteration of a small job beside a finished 128x128x256 one, FP32:
+// 196 -> 143 us).
 __device__ __forceinline__ void loads_issued() { asm volatile("" ::: "memory"); }
 
 // Element at a wavefront-uniform address plus a lane's 32-bit byte offset (the
@@ -232,7 +236,7 @@ __device__ __forceinline__ T& lane_at(T* uniform, uint32_t bytes)
 // doubled row has Dx = 2M reals, so packed complex z[n] = (x[2n], x[2n+1])
 // is non-zero only for n < M/2.
 // ---------------------------------------------------------------------------
-template <typename R, int M>
+template <typename R, int M, bool SERVED>
 __global__ __launch_bounds__(kThreads) void k_x_r2c(const GridJob* __restrict__ jobs,
                                                     const typename cplx<R>::type* __restrict__ twM,
                                                     const typename cplx<R>::type* __restrict__ tw2M,
@@ -247,6 +251,7 @@ __global__ __launch_bounds__(kThreads) void k_x_r2c(const GridJob* __restrict__ 
     T2* __restrict__ S = in_memory(static_cast<T2*>(J.S));
     const DomainRec* dom = in_memory(J.dom);
     const int error = dom->error;
+    if (SERVED && error) return;
     const int r0 = blockIdx.x * NL;
     const int Hx = M + 1;
     // precision form: the unit-weight density is scaled to unit peak here,
@@ -306,7 +311,7 @@ __global__ __launch_bounds__(kThreads) void k_x_r2c(const GridJob* __restrict__ 
 // Z'[k] = A + i conj(w^k) B, A = X[k] + conj X[M-k], B = X[k] - conj X[M-k];
 // z = inverse FFT_M(Z'); x[2n] = Re z[n], x[2n+1] = Im z[n]; keep n < M/2.
 // ---------------------------------------------------------------------------
-template <typename R, int M>
+template <typename R, int M, bool SERVED>
 __global__ __launch_bounds__(kThreads) void k_x_c2r(const GridJob* __restrict__ jobs,
                                                     const typename cplx<R>::type* __restrict__ twM,
                                                     const typename cplx<R>::type* __restrict__ tw2M,
@@ -321,6 +326,7 @@ __global__ __launch_bounds__(kThreads) void k_x_c2r(const GridJob* __restrict__ 
     R* __restrict__ phi = in_memory(static_cast<R*>(J.phi));
     const DomainRec* dom = in_memory(J.dom);
     const int error = dom->error;
+    if (SERVED && error) return;
     const int r0 = blockIdx.x * NL;
     const int Hx = M + 1;
     constexpr int K = NL * M / kThreads;
@@ -512,7 +518,7 @@ template <int L, typename T2> struct RegLines {
 // non-zero half p < L/2; 1: inverse, stores the kept half p < L/2; 2 (the z
 // pass): forward, multiply by the real Green's spectrum, inverse, half
 // loaded and half stored.
-template <typename R, int L, int MODE>
+template <typename R, int L, int MODE, bool SERVED>
 __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) void k_cols_reg(
     const GridJob* __restrict__ jobs, const typename cplx<R>::type* __restrict__ tw, int nlines,
     int lpp, int64_t plane_stride, int64_t pstride, int gy, int Hx)
@@ -527,6 +533,7 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     T2* __restrict__ S_ = in_memory(static_cast<T2*>(J.S));
     const DomainRec* dom = in_memory(J.dom);
     const int error = dom->error;
+    if (SERVED && error) return;
     const int line = int(threadIdx.x) % NL, j = int(threadIdx.x) / NL;
     const int l = xcd_group() * NL + line;
     const bool live = l < nlines;
@@ -644,7 +651,7 @@ __device__ __forceinline__ auto sin_2pi(const T2* __restrict__ tw, int k, int L)
 // line buffer.  y': the three inverse transforms likewise.  Every load of a
 // line precedes the barrier of its first exchange, so the in-place stores
 // cannot overtake a load (L <= 16: one thread per line).
-template <typename R, int L>
+template <typename R, int L, bool SERVED>
 __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) void k_z_field_reg(
     const GridJob* __restrict__ jobs, const typename cplx<R>::type* __restrict__ tw, int nlines,
     int gy, int Hx)
@@ -661,6 +668,7 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     const R* __restrict__ ghat = in_memory(static_cast<const R*>(J.ghat));
     const DomainRec* dom = in_memory(J.dom);
     const int error = dom->error;
+    if (SERVED && error) return;
     const R ihz = R(dom->inv_h[2]);
     const int line = int(threadIdx.x) % NL, j = int(threadIdx.x) / NL;
     const int l = xcd_group() * NL + line;
@@ -724,7 +732,7 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads)) voi
     }
 }
 
-template <typename R, int L>
+template <typename R, int L, bool SERVED>
 __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads), 4) void k_y_field_reg(
     const GridJob* __restrict__ jobs, const typename cplx<R>::type* __restrict__ tw, int nlines,
     int gy, int Hx)
@@ -740,6 +748,7 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads), 4) 
     T2* __restrict__ S2 = in_memory(static_cast<T2*>(J.S2));
     const DomainRec* dom = in_memory(J.dom);
     const int error = dom->error;
+    if (SERVED && error) return;
     const R ihy = R(dom->inv_h[1]);
     const int line = int(threadIdx.x) % NL, j = int(threadIdx.x) / NL;
     const int l = xcd_group() * NL + line;
@@ -794,7 +803,7 @@ __global__ __launch_bounds__((RegLines<L, typename cplx<R>::type>::threads), 4) 
     }
 }
 
-template <typename R, int M>
+template <typename R, int M, bool SERVED>
 __global__ __launch_bounds__(kThreads) void k_x_field(
     const GridJob* __restrict__ jobs, const typename cplx<R>::type* __restrict__ twM,
     const typename cplx<R>::type* __restrict__ tw2M, int gy, int gz, int Dy)
@@ -810,6 +819,7 @@ __global__ __launch_bounds__(kThreads) void k_x_field(
     T4* __restrict__ E = in_memory(static_cast<T4*>(J.E));
     const DomainRec* dom = in_memory(J.dom);
     const int error = dom->error;
+    if (SERVED && error) return;
     const R ihx = R(dom->inv_h[0]);
     const int nrows = gz * gy;
     const int r0 = blockIdx.x * NL;
@@ -1089,14 +1099,14 @@ void launch_green(const Geometry& g, int green_fn, const GridJob* jobs, int nj,
     else any_green_cols<R>(g, 2, jobs, nj, tw, st);
 }
 
-template <typename R> struct SolveX {
+template <typename R, bool SERVED> struct SolveX {
     using T2 = typename cplx<R>::type;
     template <int M> struct Fwd {
         static void run(const Geometry& g, const GridJob* jobs, int nj, const T2* tw,
                         hipStream_t st)
         {
             int rows = g.gz * g.gy;
-            hipLaunchKernelGGL((k_x_r2c<R, M>), dim3(nblocks(rows, XLines<M>::value), nj),
+            hipLaunchKernelGGL((k_x_r2c<R, M, SERVED>), dim3(nblocks(rows, XLines<M>::value), nj),
                                dim3(kThreads), 0, st, jobs, tw + twiddle_offset(M),
                                tw + twiddle_offset(2 * M), rows, g.gy, g.Dy);
         }
@@ -1106,7 +1116,7 @@ template <typename R> struct SolveX {
                         hipStream_t st)
         {
             int rows = g.gz * g.gy;
-            hipLaunchKernelGGL((k_x_c2r<R, M>), dim3(nblocks(rows, XLines<M>::value), nj),
+            hipLaunchKernelGGL((k_x_c2r<R, M, SERVED>), dim3(nblocks(rows, XLines<M>::value), nj),
                                dim3(kThreads), 0, st, jobs, tw + twiddle_offset(M),
                                tw + twiddle_offset(2 * M), rows, g.gy, g.Dy);
         }
@@ -1116,7 +1126,7 @@ template <typename R> struct SolveX {
                         hipStream_t st)
         {
             int lines = g.gz * g.Hx;
-            hipLaunchKernelGGL((k_cols_reg<R, L, 0>),
+            hipLaunchKernelGGL((k_cols_reg<R, L, 0, SERVED>),
                                dim3(col_blocks(lines, RegLines<L, T2>::value), nj),
                                dim3(RegLines<L, T2>::threads), 0, st, jobs, tw + twiddle_offset(L),
                                lines, g.Hx, int64_t(g.Dy) * g.Hx, int64_t(g.Hx), g.gy, g.Hx);
@@ -1127,7 +1137,7 @@ template <typename R> struct SolveX {
                         hipStream_t st)
         {
             int lines = g.gz * g.Hx;
-            hipLaunchKernelGGL((k_cols_reg<R, L, 1>),
+            hipLaunchKernelGGL((k_cols_reg<R, L, 1, SERVED>),
                                dim3(col_blocks(lines, RegLines<L, T2>::value), nj),
                                dim3(RegLines<L, T2>::threads), 0, st, jobs, tw + twiddle_offset(L),
                                lines, g.Hx, int64_t(g.Dy) * g.Hx, int64_t(g.Hx), g.gy, g.Hx);
@@ -1138,7 +1148,7 @@ template <typename R> struct SolveX {
                         hipStream_t st)
         {
             int lines = g.Dy * g.Hx;
-            hipLaunchKernelGGL((k_cols_reg<R, L, 2>),
+            hipLaunchKernelGGL((k_cols_reg<R, L, 2, SERVED>),
                                dim3(col_blocks(lines, RegLines<L, T2>::value), nj),
                                dim3(RegLines<L, T2>::threads), 0, st, jobs, tw + twiddle_offset(L),
                                lines, lines, int64_t(0), int64_t(lines), g.gy, g.Hx);
@@ -1149,7 +1159,7 @@ template <typename R> struct SolveX {
                         hipStream_t st)
         {
             int lines = g.Dy * g.Hx;
-            hipLaunchKernelGGL((k_z_field_reg<R, L>),
+            hipLaunchKernelGGL((k_z_field_reg<R, L, SERVED>),
                                dim3(col_blocks(lines, RegLines<L, T2>::value), nj),
                                dim3(RegLines<L, T2>::threads), 0, st, jobs, tw + twiddle_offset(L),
                                lines, g.gy, g.Hx);
@@ -1160,7 +1170,7 @@ template <typename R> struct SolveX {
                         hipStream_t st)
         {
             int lines = g.gz * g.Hx;
-            hipLaunchKernelGGL((k_y_field_reg<R, L>),
+            hipLaunchKernelGGL((k_y_field_reg<R, L, SERVED>),
                                dim3(col_blocks(lines, RegLines<L, T2>::value), nj),
                                dim3(RegLines<L, T2>::threads), 0, st, jobs, tw + twiddle_offset(L),
                                lines, g.gy, g.Hx);
@@ -1171,7 +1181,7 @@ template <typename R> struct SolveX {
                         hipStream_t st)
         {
             int rows = g.gz * g.gy;
-            hipLaunchKernelGGL((k_x_field<R, M>),
+            hipLaunchKernelGGL((k_x_field<R, M, SERVED>),
                                dim3(nblocks(rows, RowLines<M, 3, T2>::value), nj),
                                dim3(kThreads), 0, st, jobs, tw + twiddle_offset(M),
                                tw + twiddle_offset(2 * M), g.gy, g.gz, g.Dy);
@@ -1179,45 +1189,59 @@ template <typename R> struct SolveX {
     };
 };
 
-template <typename R>
-void launch_solve(const Geometry& g, const GridJob* jobs, int nj,
+template <typename R, bool SERVED>
+static void solve(const Geometry& g, const GridJob* jobs, int nj,
                   const typename cplx<R>::type* tw, hipStream_t st)
 {
-    if (g.tuned[0]) dispatch_len<SolveX<R>::template Fwd>(g.gx, g, jobs, nj, tw, st);
+    if (g.tuned[0]) dispatch_len<SolveX<R, SERVED>::template Fwd>(g.gx, g, jobs, nj, tw, st);
     else any_x_pass<R>(g, false, jobs, nj, tw, st);
-    if (g.tuned[1]) dispatch_len<SolveX<R>::template YFwd>(g.Dy, g, jobs, nj, tw, st);
+    if (g.tuned[1]) dispatch_len<SolveX<R, SERVED>::template YFwd>(g.Dy, g, jobs, nj, tw, st);
     else any_cols<R>(g, 0, jobs, nj, tw, st);
-    if (g.tuned[2]) dispatch_len<SolveX<R>::template ZConv>(g.Dz, g, jobs, nj, tw, st);
+    if (g.tuned[2]) dispatch_len<SolveX<R, SERVED>::template ZConv>(g.Dz, g, jobs, nj, tw, st);
     else any_cols<R>(g, 2, jobs, nj, tw, st);
-    if (g.tuned[1]) dispatch_len<SolveX<R>::template YInv>(g.Dy, g, jobs, nj, tw, st);
+    if (g.tuned[1]) dispatch_len<SolveX<R, SERVED>::template YInv>(g.Dy, g, jobs, nj, tw, st);
     else any_cols<R>(g, 1, jobs, nj, tw, st);
-    if (g.tuned[0]) dispatch_len<SolveX<R>::template Inv>(g.gx, g, jobs, nj, tw, st);
+    if (g.tuned[0]) dispatch_len<SolveX<R, SERVED>::template Inv>(g.gx, g, jobs, nj, tw, st);
     else any_x_pass<R>(g, true, jobs, nj, tw, st);
 }
 
-template <typename R>
-void launch_solve_field(const Geometry& g, const GridJob* jobs, int nj,
+template <typename R, bool SERVED>
+static void solve_field(const Geometry& g, const GridJob* jobs, int nj,
                         const typename cplx<R>::type* tw, hipStream_t st)
 {
-    if (g.tuned[0]) dispatch_len<SolveX<R>::template Fwd>(g.gx, g, jobs, nj, tw, st);
+    if (g.tuned[0]) dispatch_len<SolveX<R, SERVED>::template Fwd>(g.gx, g, jobs, nj, tw, st);
     else any_x_pass<R>(g, false, jobs, nj, tw, st);
-    if (g.tuned[1]) dispatch_len<SolveX<R>::template YFwd>(g.Dy, g, jobs, nj, tw, st);
+    if (g.tuned[1]) dispatch_len<SolveX<R, SERVED>::template YFwd>(g.Dy, g, jobs, nj, tw, st);
     else any_cols<R>(g, 0, jobs, nj, tw, st);
-    if (g.tuned[2]) dispatch_len<SolveX<R>::template ZField>(g.Dz, g, jobs, nj, tw, st);
+    if (g.tuned[2]) dispatch_len<SolveX<R, SERVED>::template ZField>(g.Dz, g, jobs, nj, tw, st);
     else any_field<R>(g, 0, jobs, nj, tw, st);
-    if (g.tuned[1]) dispatch_len<SolveX<R>::template YField>(g.Dy, g, jobs, nj, tw, st);
+    if (g.tuned[1]) dispatch_len<SolveX<R, SERVED>::template YField>(g.Dy, g, jobs, nj, tw, st);
     else any_field<R>(g, 1, jobs, nj, tw, st);
-    if (g.tuned[0]) dispatch_len<SolveX<R>::template XField>(g.gx, g, jobs, nj, tw, st);
+    if (g.tuned[0]) dispatch_len<SolveX<R, SERVED>::template XField>(g.gx, g, jobs, nj, tw, st);
     else any_field<R>(g, 2, jobs, nj, tw, st);
+}
+
+template <typename R>
+void launch_solve(const Geometry& g, const GridJob* jobs, int nj, bool served,
+                  const typename cplx<R>::type* tw, hipStream_t st)
+{
+    served ? solve<R, true>(g, jobs, nj, tw, st) : solve<R, false>(g, jobs, nj, tw, st);
+}
+
+template <typename R>
+void launch_solve_field(const Geometry& g, const GridJob* jobs, int nj, bool served,
+                        const typename cplx<R>::type* tw, hipStream_t st)
+{
+    served ? solve_field<R, true>(g, jobs, nj, tw, st) : solve_field<R, false>(g, jobs, nj, tw, st);
 }
 
 template void launch_green<double>(const Geometry&, int, const GridJob*, int, const double2*,
                                    hipStream_t);
 template void launch_green<float>(const Geometry&, int, const GridJob*, int, const float2*,
                                   hipStream_t);
-template void launch_solve<double>(const Geometry&, const GridJob*, int, const double2*,
+template void launch_solve<double>(const Geometry&, const GridJob*, int, bool, const double2*,
                                    hipStream_t);
-template void launch_solve_field<float>(const Geometry&, const GridJob*, int, const float2*,
+template void launch_solve_field<float>(const Geometry&, const GridJob*, int, bool, const float2*,
                                         hipStream_t);
 
 }  // namespace sc3d

@@ -103,14 +103,14 @@ void launch_green(const Geometry& g, int green_fn, const GridJob* jobs, int nj,
 
 // FP64 form: rho -> phi (five passes, convolution fused into the z pass).
 template <typename R>
-void launch_solve(const Geometry& g, const GridJob* jobs, int nj,
+void launch_solve(const Geometry& g, const GridJob* jobs, int nj, bool served,
                   const typename cplx<R>::type* tw, hipStream_t st);
 
 // Precision form: the same convolution, with the field transformed straight
 // from the spectrum (E = IDFT(phi^ * D_a), D_a = -i sin(2 pi k/D_a)/h_a) and
 // written as (Ex, Ey, Ez, 0) per node.  No potential is formed.
 template <typename R>
-void launch_solve_field(const Geometry& g, const GridJob* jobs, int nj,
+void launch_solve_field(const Geometry& g, const GridJob* jobs, int nj, bool served,
                         const typename cplx<R>::type* tw, hipStream_t st);
 
 // The generic passes (sc3d_fft_any.hip) of the axes whose lengths the tuned

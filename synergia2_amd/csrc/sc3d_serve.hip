@@ -203,6 +203,7 @@ int admit_alloc(sc3d_server* s, Job* j)
     const int64_t n = sp.n_particles;
     const sc3d_options o = job_options(sp, s->opt.precision, s->opt.sort_period);
     if (int rc = sc3d_create(&o, &j->ctx)) return rc;
+    j->ctx->served = true;
     // one allocation for the job's own buffers, 256-byte aligned each
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
     const size_t b_parts = up(size_t(n) * 7 * sizeof(double)), b_masks = up(size_t(n)),
