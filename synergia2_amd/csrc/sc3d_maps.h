@@ -156,10 +156,12 @@ struct MapProgram {
 //      ulp: that is its seed, and s/(2 |l| C) the slope, for one residual step.
 //      Signed by l, so no separate sign multiplication.
 // The last step needs |l| C / s accurate to a few ulp, so a in [1/2, 2] (no
-// cancellation; a particle outside takes drift_unit) and 1/beta^2 away from 1
-// (at 1 and |l| near a power of two D2/beta^2 comes next to a power of four,
-// where one residual step cannot decide the rounding; there the path length
-// has a square root of its own).
+// cancellation) and 1/beta^2 away from 1 (at 1 and |l| near a power of two
+// D2/beta^2 comes next to a power of four, where one residual step cannot
+// decide the rounding).  A wavefront with a particle outside takes the rolled
+// form for all its particles, whose path length has a square root of its own
+// (any a >= 2^-100); what that form cannot hold either (a <= 0, NaN, `ones`)
+// takes drift_unit.
 // Measured (4e6 particles, mean over the 10 steps of an O-F-O-D cell, 6
 // quadrupole slices among them): maps pass 266 -> 172 us, kick with maps fused
 // (whole step) 449 -> 364 us; a step of drifts alone stays at 54 us, its
@@ -168,6 +170,7 @@ struct MapProgram {
 // took the kernel to 156 VGPRs.
 // ---------------------------------------------------------------------------
 constexpr int32_t kHighOfHalf = 0x3fe00000;  // high word of 0.5
+constexpr int32_t kHighOfTiny = 0x39b00000;  // ... of 2^-100
 constexpr double kNearLight = 1.0 + 1.0e-6;  // 1/beta^2, see above
 
 struct FastDrift {
@@ -195,7 +198,7 @@ __device__ __forceinline__ bool fast_begin(FastDrift& f, double dpop, double ref
     f.half_rc = 0.5 / f.c;
     f.a_low = INT32_MAX;
     f.ones = 0u;
-    return dp > 0.0 && f.dp2 <= 2.0 && f.ibeta2 >= 1.0 && f.ibeta2 < 1.0e12;
+    return dp > 0.0 && f.dp2 <= 1.0e60 && f.ibeta2 >= 1.0 && f.ibeta2 < 1.0e12;
 }
 
 __device__ __forceinline__ double fast_a(FastDrift& f, double xp, double yp)
@@ -203,11 +206,6 @@ __device__ __forceinline__ double fast_a(FastDrift& f, double xp, double yp)
     const double a = f.dp2 - xp * xp - yp * yp;
     f.a_low = min(f.a_low, int32_t(__double_as_longlong(a) >> 32));
     return a;
-}
-
-__device__ __forceinline__ bool fast_held(const FastDrift& f)
-{
-    return f.a_low >= kHighOfHalf && f.ones != 0xffffffffu;
 }
 
 // drift_unit over length l (l2 = l*l); kl ~ l C, hl ~ 1 / (2 l C).  OWN_ROOT:
@@ -277,9 +275,10 @@ __device__ __forceinline__ void fast_quad(FastDrift& f, const PreparedSlice& s, 
     }
 }
 
-// The same with a skew strength, and next to the speed of light; rolled: a
-// second unrolled form does not fit the 128 registers (740 us where
-// the unrolled one takes 505 and the general one 1000; 4e6 particles, O-F-O-D).
+// The same with a skew strength, next to the speed of light and for wide
+// bunches; rolled: a second unrolled form does not fit the 128 registers (740 us
+// where the unrolled one takes 505 and the general one 1000; 4e6 particles,
+// O-F-O-D).
 __device__ __forceinline__ void fast_quad_rolled(FastDrift& f, const PreparedSlice& s, double& x,
                                                  double& xp, double& y, double& yp, double& cdt)
 {
@@ -297,10 +296,10 @@ __device__ __forceinline__ void fast_quad_rolled(FastDrift& f, const PreparedSli
     }
 }
 
-__device__ __forceinline__ void fast_slice_apply(FastDrift& f, const PreparedSlice& s, double& x,
-                                                 double& xp, double& y, double& yp, double& cdt)
+__device__ __forceinline__ void fast_slice_apply(FastDrift& f, const PreparedSlice& s,
+                                                 bool rolled, double& x, double& xp, double& y,
+                                                 double& yp, double& cdt)
 {
-    const bool rolled = f.ibeta2 <= kNearLight;
     const double l = s.length;
     if (s.kind == SC3D_MAP_DRIFT) {
         if (l == 0.0) {
@@ -319,9 +318,10 @@ __device__ __forceinline__ void fast_slice_apply(FastDrift& f, const PreparedSli
     }
 }
 
-// The whole program on one particle: the fast form, and for a particle that
-// left its range the general one from the start state, which `again` brings
-// back (re-read rather than held: 10 registers over the fast loop).
+// The whole program on one particle: the fast form; in a wavefront with a
+// particle out of its range (tested after every slice) the rolled form from the
+// start state, which `again` brings back (re-read rather than held: 10
+// registers over the fast loop); the general form for what is left.
 template <typename Again>
 __device__ __forceinline__ void apply_program(const MapProgram& prog, double& x, double& xp,
                                               double& y, double& yp, double& cdt, double dpop,
@@ -332,8 +332,22 @@ __device__ __forceinline__ void apply_program(const MapProgram& prog, double& x,
     if (fast) {
         FastDrift f;
         if (fast_begin(f, dpop, prog.ref_p, prog.mass)) {
-            for (int k = 0; k < prog.n; ++k) fast_slice_apply(f, prog.s[k], x, xp, y, yp, cdt);
-            if (fast_held(f)) return;
+            // uniform over the lanes in here
+            bool rolled = __any(f.ibeta2 <= kNearLight || f.dp2 > 2.0);
+            int k;
+            for (;;) {
+                for (k = 0; k < prog.n; ++k) {
+                    fast_slice_apply(f, prog.s[k], rolled, x, xp, y, yp, cdt);
+                    if (!rolled && __any(f.a_low < kHighOfHalf)) break;
+                }
+                if (k == prog.n || __any(f.a_low < kHighOfTiny)) break;
+                again();
+                f.a_low = INT32_MAX;
+                f.ones = 0u;
+                rolled = true;
+            }
+            const bool held = k == prog.n && f.a_low >= kHighOfTiny && f.ones != 0xffffffffu;
+            if (held) return;
             again();
         }
     }
