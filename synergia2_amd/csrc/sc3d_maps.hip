@@ -95,11 +95,17 @@ int sc3d_apply_maps(const sc3d_bunch* b, const sc3d_map_slice* slices, int nslic
     prog.n = nslices;
     prog.ref_p = b->ref_p;
     prog.mass = b->mass;
-    const int64_t blocks = (n + sc3d::kThreads - 1) / sc3d::kThreads;
-    hipLaunchKernelGGL(sc3d::k_maps, dim3(unsigned(blocks)), dim3(sc3d::kThreads), 0,
-                       static_cast<hipStream_t>(stream), b->parts, b->stride, b->masks, n, prog);
-    if (hipGetLastError() != hipSuccess)
-        return sc3d_internal_fail(SC3D_ERR_HIP, "sc3d_apply_maps: launch failed");
+    // one thread per particle, and a launch takes fewer than 2^32 threads
+    constexpr int64_t kLaunch = int64_t(1) << 31;
+    for (int64_t at = 0; at < n; at += kLaunch) {
+        const int64_t part = n - at < kLaunch ? n - at : kLaunch;
+        const int64_t blocks = (part + sc3d::kThreads - 1) / sc3d::kThreads;
+        hipLaunchKernelGGL(sc3d::k_maps, dim3(unsigned(blocks)), dim3(sc3d::kThreads), 0,
+                           static_cast<hipStream_t>(stream), b->parts + at, b->stride,
+                           b->masks + at, part, prog);
+        if (hipGetLastError() != hipSuccess)
+            return sc3d_internal_fail(SC3D_ERR_HIP, "sc3d_apply_maps: launch failed");
+    }
     return SC3D_OK;
 }
 
