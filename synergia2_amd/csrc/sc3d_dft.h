@@ -145,12 +145,6 @@ __device__ __forceinline__ void dft_small(T2* v)
         dft_coprime<2, 3, INV>(v);
     } else if constexpr (R == 10) {
         dft_coprime<2, 5, INV>(v);
-    } else if constexpr (R == 12) {
-        dft_coprime<4, 3, INV>(v);
-    } else if constexpr (R == 14) {
-        dft_coprime<2, 7, INV>(v);
-    } else if constexpr (R == 15) {
-        dft_coprime<3, 5, INV>(v);
     } else if constexpr (R == 9) {
         // 3 x 3 with the twiddles w^1, w^2, w^4, w = e^(-2 pi i / 9)
         using F = decltype(v[0].x);

@@ -96,11 +96,11 @@ template <typename T2> constexpr bool any_table() { return sizeof(T2) < 16; }
 // Butterflies of radix r of one thread in a pass: about ten elements held (four
 // wavefronts per SIMD; three radix-4 or radix-5 table butterflies spill).
 constexpr int any_per(int r) { return r <= 3 ? 3 : (r <= 5 ? 2 : 1); }
-// Radices with a register butterfly; the others (primes) go one output per
-// thread.  Table butterflies of a composite radix are two consecutive passes,
+// Radices with a register butterfly (FP64 2..11 and 13, FP32 2..10, 12 and 16;
+// 14 and 15 as well spilled, and the scratch slowed every radix: 96x80x150 526
+// -> 596 us a step); larger primes (FP32: from 11) go one output per thread.
+// Table butterflies of a composite radix are two consecutive passes,
 // any_split(r) then r / any_split(r), on the elements of one thread.
-// (14 and 15 spill, and the scratch slows every radix: 96x80x150 526 -> 596 us
-// a step.)
 constexpr int any_split(int r)
 {
     return r == 8 || r == 12 || r == 16 ? 4 : (r == 6 || r == 10 ? 2 : (r == 9 ? 3 : r));
@@ -130,8 +130,6 @@ template <typename T2, typename F> __device__ __forceinline__ void with_radix(in
         SC3D_ANY_RADIX(11)
         SC3D_ANY_RADIX(12)
         SC3D_ANY_RADIX(13)
-        SC3D_ANY_RADIX(14)
-        SC3D_ANY_RADIX(15)
         SC3D_ANY_RADIX(16)
 #undef SC3D_ANY_RADIX
     }
