@@ -1186,8 +1186,10 @@ inline int64_t nblk(int64_t items, int per) { return (items + per - 1) / per; }
 
 // Blocks of the passes: lines (or pairs) in groups of K transforms.
 // Columns: runs of 128 bytes over neighbouring lines; rows: 256 threads.
-// Fewer where the threads or the LDS pass their bounds (40 KiB keeps four
-// blocks on a CU; one line always fits 64 KiB).
+// Fewer where the threads or the LDS pass their bounds (three blocks on a CU's
+// 160 KiB; 40 KiB for four made no difference); one line always fits the 64 KiB
+// of a block.
+constexpr size_t kAnyLds = 53000;
 template <typename T2> AnyShape any_shape(const AnyPlan& pl, int K, bool rows, size_t& lds)
 {
     AnyShape a{};
@@ -1202,7 +1204,7 @@ template <typename T2> AnyShape any_shape(const AnyPlan& pl, int K, bool rows, s
     // (at most ceil(1022 / 2 / 3) = 171 threads: one line always fits)
     a.tpl = direct ? std::max(pl.tpl, std::min(pl.L / 4, kAnyPreferred / K)) : pl.tpl;
     a.nl = rows ? std::min(16, std::max(1, 256 / (a.tpl * K))) : 128 / int(sizeof(T2));
-    while (a.nl > 1 && (a.nl * K * a.tpl > kAnyPreferred || bytes(a.nl) > 53000)) a.nl /= 2;
+    while (a.nl > 1 && (a.nl * K * a.tpl > kAnyPreferred || bytes(a.nl) > kAnyLds)) a.nl /= 2;
     a.lines = a.nl * K;
     lds = bytes(a.nl);
     return a;
