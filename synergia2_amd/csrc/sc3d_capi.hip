@@ -261,9 +261,9 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
     a.ref_beta = b->ref_beta;
     // The bunch storage is cell-sorted (sort + reorder) every sort_period
     // applies (served form: on the iterations the server picks, sc.sort_now);
-    // the deposit then works on windows of the storage, sorted by cell in
-    // LDS.  sort_period 0 never reorders: the sort then runs on every apply
-    // and the deposit walks its permutation.
+    // the deposit then works on windows of the storage.  sort_period 0 never
+    // reorders: the sort then runs on every apply and the deposit walks its
+    // permutation.
     const bool local_dep = o.sort_period > 0;
     const bool do_reorder =
         n > 0 && local_dep &&

@@ -92,8 +92,9 @@ int64_t test_alloc_limit();
 
 // Several buffers of one lifetime in one device allocation (each 256-byte
 // aligned): a context's buffers cost one hipMalloc and one hipFree instead of
-// ten, and hipFree waits for the device each time (eight served jobs: 205 pairs
-// and 47.5 ms before, 33.7 ms now).  The test limit applies to each buffer.
+// ten, and hipFree waits for the device each time (a pass of eight served jobs:
+// with 205 pairs 51.0 ms, with the merged ones, the jobs' own buffers among
+// them, 39.2, the same kernels).  The test limit applies to each buffer.
 class BufferSet {
 public:
     template <typename T>

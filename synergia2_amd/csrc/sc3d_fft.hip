@@ -70,6 +70,9 @@ template <int L> struct HalfLines {
 // serial function, and 7 lines waste less of the last round than 8 (32x32x64
 // FP64, 32 -> 7 lines: 68 -> 307 blocks, 7.7 -> 4.6 us; 64x64x128, 16 -> 7:
 // FP64 13.2 -> 11.8, FP32 11.6 -> 10.2; 128x128x256 FP32, 8 -> 7: 45.3 -> 46.5).
+// For the shortest rows 28 and 15 lines and 7 are alike (all three Green's
+// passes, FP64: 8x64x128 128 / 28 / 7 lines 18.5 / 15.4 / 15.6 us, 16x16x32 64 /
+// 15 / 7 lines 17.3 / 13.8 / 13.7).
 template <int M> struct GreenXLines {
     static constexpr int value = M == 8 ? 28 : M == 16 ? 15 : M <= 64 ? 7 : 8;
 };

@@ -64,8 +64,11 @@ void launch_sort(const double* parts, int64_t stride, const uint8_t* masks, int6
 void launch_reorder(double* parts, int64_t stride, uint8_t* masks, int64_t n, const int32_t* perm,
                     double* scratch, uint8_t* smask, const DomainRec* dom, hipStream_t st);
 // Reorder in place, for a storage in unknown order; scratch and smask are used.
-// From kRecordReorder particles on (below, the bunch stays in the caches: 1e5
-// particles 11.6 us against 7.8).
+// From kRecordReorder particles on (below, the bunch stays in the caches).  Sort
+// and kick of a first apply on a bunch in random order, launch_reorder / this,
+// us: 5e4 particles 52 / 53, 1e5 58 / 58, 2e5 73 / 66, 2.5e5 80 / 69, 3e5 90 / 75,
+// 6e5 146 / 103; in a storage already sorted this is the slower one (1.6e7:
+// +400), so the line lies above where the two meet.
 constexpr int64_t kRecordReorder = 250000;
 void launch_reorder_records(double* parts, int64_t stride, uint8_t* masks, int64_t n,
                             const int32_t* perm, double* scratch, uint8_t* smask,

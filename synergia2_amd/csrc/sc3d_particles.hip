@@ -1957,7 +1957,7 @@ static void launch_deposit_tiles(const double* parts, int64_t stride, const uint
     // phase at 1 / 2 / 4 slots, us: 1e4 particles 8.6 / 9.8 / 14.9, 1e5 8.4 / 9.1
     // / 11.6 on 32x32x64; 4e5 on 64x64x128 14.8 / 12.6 / 15.5; 1e6 23.4 / 20.6 /
     // 19.9); one through a permutation, whose random reads want the wavefronts
-    // (2e6 122 / 125 / 127, 4e6 266 / 273 / 279).
+    // (1e5 11.1 / 12.4 / 18.0, 1e6 25.2 / 25.8 / 31.6, 4e6 82.8 / 81.8 / 84.1).
     if (perm != nullptr)
         launch(k_deposit_tile<UNIT, 1, true>, 1);
     else if (n < 250000)
