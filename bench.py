@@ -713,7 +713,7 @@ def measured_traffic(config):
         doc = json.load(f)
     out = {}
     for name, rec in doc["kernels"].items():
-        if "k_kick_tile<" in name and ", false>" in name:  # not the reordering apply's
+        if "k_kick_tile<" in name and ", false," in name:  # not the reordering apply's
             out["k_kick_tile"] = rec["traffic_bytes"]
         elif "k_deposit_tile<" in name:
             out["k_deposit_tile"] = rec["traffic_bytes"]
