@@ -934,10 +934,13 @@ __global__ void k_fill(R* __restrict__ p, int64_t n, R v)
 // windows lie at the two ends of the cell order (the tails of the bunch), so
 // the block order is rotated to start the last eighth of the windows
 // first and keep them off the end of the kernel.  Tile and grid accumulate in
-// FP64 for both precisions; the precision form's unit-weight sums are rounded
-// once, by k_rho_round.  (Global adds in FP32 left each node an order-dependent
-// error of 6e-8; over a few steps that moved single particles across a cell
-// face, and so the slots of the next reorder, from one run to the next.)
+// FP64 for both precisions; the precision form's unit weights are rounded to
+// FP32 once per node and window, as they leave the tile, and their sum once
+// more, by k_rho_round: FP64 holds the sums of FP32 values exactly, so the
+// order of the global adds does not matter.  (Added in FP32 it left a node an
+// error of up to 6e-8 per window; over a few steps that moved single particles
+// across a cell face, and so the slots of the next reorder, from one run to the
+// next.)
 // Measured against the windowed kernel it replaces (LDS radix sort of each
 // window, lane runs, DPP segmented scan, LDS run list; PMC: 465 VALU
 // instructions per particle), deposit phase per step over sort periods of
@@ -1065,8 +1068,15 @@ __device__ __forceinline__ void tile_deposit(double* tile, int bx, int by, int b
     if (cur >= 0) add();
 }
 
+// What the window adds to a node.
+template <bool UNIT> __device__ __forceinline__ double grid_sum(double v)
+{
+    return UNIT ? double(float(v)) : v;
+}
+
 // The non-zero interior nodes of a tile (box at (bx, by, bz), nx x ny x ..,
 // `nodes` in all) into rho, node e of the thread's share first..step.
+template <bool UNIT>
 __device__ __forceinline__ void tile_flush(const double* tile, int nodes, int first, int step,
                                            int bx, int by, int bz, int nx, int ny, int gx, int gy,
                                            int gz, double* __restrict__ rho)
@@ -1078,7 +1088,7 @@ __device__ __forceinline__ void tile_flush(const double* tile, int nodes, int fi
         const int r = small_div(e, mx), rz = small_div(r, my);
         const int cx = bx + e - r * nx, cy = by + r - rz * ny, cz = bz + rz;
         if (cx > 0 && cx < gx - 1 && cy > 0 && cy < gy - 1 && cz > 0 && cz < gz - 1)
-            unsafeAtomicAdd(rho + (int64_t(cz) * gy + cy) * gx + cx, v);
+            unsafeAtomicAdd(rho + (int64_t(cz) * gy + cy) * gx + cx, grid_sum<UNIT>(v));
     }
 }
 
@@ -1192,7 +1202,8 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
         __syncthreads();
         tile_deposit(tile, blo[0], blo[1], blo[2], nx, ny, lc, w0, ix, iy, iz, ok, ox, oy, oz);
         __syncthreads();
-        tile_flush(tile, nodes, t, kTileThreads, blo[0], blo[1], blo[2], nx, ny, gx, gy, gz, rho);
+        tile_flush<UNIT>(tile, nodes, t, kTileThreads, blo[0], blo[1], blo[2], nx, ny, gx, gy, gz,
+                         rho);
         return;
     }
     // the window's box does not fit: this wavefront's own box in its quarter
@@ -1207,7 +1218,7 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
         tile_deposit(wtile, lo[0], lo[1], lo[2], wnx, wny, lc, w0, ix, iy, iz, ok, ox, oy, oz);
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        tile_flush(wtile, wn, lane, 64, lo[0], lo[1], lo[2], wnx, wny, gx, gy, gz, rho);
+        tile_flush<UNIT>(wtile, wn, lane, 64, lo[0], lo[1], lo[2], wnx, wny, gx, gy, gz, rho);
         return;
     }
     // scattered particles (the sparse tails, or a storage out of cell order):
@@ -1227,10 +1238,9 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
     for (int q = 0; q < PER; ++q) {
         if (!ok[q]) continue;
         double w[8];
-        lc.weights(w0, ox[q], oy[q], oz[q], w);
+        LaneCorners(0).weights(w0, ox[q], oy[q], oz[q], w);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int c = k ^ (lane & 7);
+        for (int c = 0; c < 8; ++c) {
             const int cx = ix[q] + (c & 1), cy = iy[q] + ((c >> 1) & 1), cz = iz[q] + (c >> 2);
             if (!(cx > 0 && cx < gx - 1 && cy > 0 && cy < gy - 1 && cz > 0 && cz < gz - 1))
                 continue;
@@ -1238,16 +1248,16 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
             const int slot = int((uint32_t(node) * 2654435761u) >> 23) & (kCacheSlots - 1);
             const int held = atomicCAS(&ckey[slot], -1, node);
             if (held == -1 || held == node)
-                unsafeAtomicAdd(&cval[slot], w[k]);
+                unsafeAtomicAdd(&cval[slot], w[c]);
             else
-                unsafeAtomicAdd(rho + node, w[k]);
+                unsafeAtomicAdd(rho + node, grid_sum<UNIT>(w[c]));
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
     for (int e = lane; e < kCacheSlots; e += 64) {
         const int node = ckey[e];
-        if (node >= 0) unsafeAtomicAdd(rho + node, cval[e]);
+        if (node >= 0) unsafeAtomicAdd(rho + node, grid_sum<UNIT>(cval[e]));
     }
 }
 
@@ -1255,7 +1265,10 @@ __global__ __launch_bounds__(kTileThreads) void k_deposit_tile(
 // and the peak of that (all entries >= 0, so the IEEE bit patterns order like
 // the values): block max (wavefront butterflies, then LDS), one integer
 // atomicMax per block into the domain record (cleared by k_domain_finish each
-// apply); the grid is bounded so few atomics meet.
+// apply); the grid is bounded so few atomics meet, about 10 ns each on their
+// one address (128x128x256, up to 256 / 512 / 1024 / 2048 blocks of 16, 8, 8 and
+// 8 loads per round: 11.4 / 13.3 / 17.7 / 28.2 us; the peak alone, of FP32 sums,
+// took 8.7).
 __global__ __launch_bounds__(kThreads) void k_rho_round(const double* __restrict__ sums,
                                                         float* __restrict__ rho, int64_t G,
                                                         DomainRec* __restrict__ dom)
@@ -1263,15 +1276,15 @@ __global__ __launch_bounds__(kThreads) void k_rho_round(const double* __restrict
     __shared__ float wmax[kThreads / 64];
     if (dom->error) return;
     float m = 0.0f;
-    // eight independent loads in flight per lane and round
+    // sixteen independent loads in flight per lane and round
     const int64_t T = int64_t(gridDim.x) * kThreads;
     int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x;
-    for (; i + 7 * T < G; i += 8 * T) {
-        double v[8];
+    for (; i + 15 * T < G; i += 16 * T) {
+        double v[16];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = sums[i + u * T];
+        for (int u = 0; u < 16; ++u) v[u] = sums[i + u * T];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < 16; ++u) {
             const float r = float(v[u]);
             rho[i + u * T] = r;
             m = fmaxf(m, r);
@@ -1958,14 +1971,25 @@ static void launch_deposit_tiles(const double* parts, int64_t stride, const uint
     // / 11.6 on 32x32x64; 4e5 on 64x64x128 14.8 / 12.6 / 15.5; 1e6 23.4 / 20.6 /
     // 19.9); one through a permutation, whose random reads want the wavefronts
     // (1e5 11.1 / 12.4 / 18.0, 1e6 25.2 / 25.8 / 31.6, 4e6 82.8 / 81.8 / 84.1).
-    if (perm != nullptr)
+    // The precision form keeps four everywhere: its windows are the groups that
+    // are rounded together, and smaller ones move a sparse bunch's field by
+    // more than its earlier results differ among themselves (n < 60000: dp/p by
+    // 1e-8 where they differ by 2e-9).
+    if (perm != nullptr) {
         launch(k_deposit_tile<UNIT, 1, true>, 1);
-    else if (n < 250000)
-        launch(k_deposit_tile<UNIT, 1, false>, 1);
-    else if (n < 750000)
-        launch(k_deposit_tile<UNIT, 2, false>, 2);
-    else
-        launch(k_deposit_tile<UNIT, 4, false>, 4);
+        return;
+    }
+    if constexpr (!UNIT) {
+        if (n < 250000) {
+            launch(k_deposit_tile<UNIT, 1, false>, 1);
+            return;
+        }
+        if (n < 750000) {
+            launch(k_deposit_tile<UNIT, 2, false>, 2);
+            return;
+        }
+    }
+    launch(k_deposit_tile<UNIT, 4, false>, 4);
 }
 
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
@@ -1978,7 +2002,7 @@ void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
     }
     launch_deposit_tiles<true>(parts, stride, masks, perm, n, gx, gy, gz, dom, sums, st);
     const int64_t G = int64_t(gx) * gy * gz;
-    hipLaunchKernelGGL(k_rho_round, dim3(grid_for(G / 8, 512)), dim3(kThreads), 0, st, sums, rho32,
+    hipLaunchKernelGGL(k_rho_round, dim3(grid_for(G / 16, 256)), dim3(kThreads), 0, st, sums, rho32,
                        G, dom);
 }
 
