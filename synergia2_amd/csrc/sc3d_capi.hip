@@ -304,7 +304,7 @@ int enqueue_front(sc3d_ctx* c, const sc3d_bunch* b, double time_step, const Sche
     const int64_t ds = c->reordering ? n : b->stride;
     const uint8_t* dm = c->reordering ? c->smask : b->masks;
     launch_deposit(dp, ds, dm, dep_perm, n, g.gx, g.gy, g.gz, c->dom, c->sums,
-                   c->fp32 ? static_cast<float*>(c->rho) : nullptr, st);
+                   c->fp32 ? static_cast<float*>(c->rho) : nullptr, c->served, st);
     ev[3] = mark(c, st);
     return SC3D_OK;
 }

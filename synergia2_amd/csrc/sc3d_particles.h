@@ -78,10 +78,10 @@ void launch_reorder_records(double* parts, int64_t stride, uint8_t* masks, int64
 // reorder), else of the permutation `perm` of this step's sort.  sums: the
 // density, cleared (launch_domain).  rho32 non-null (precision form): unit
 // weights; k_rho_round then rounds the sums to rho32 and records the density
-// peak in the domain record.
+// peak in the domain record.  served: an apply of the served form.
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
                     const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
-                    double* sums, float* rho32, hipStream_t st);
+                    double* sums, float* rho32, bool served, hipStream_t st);
 template <typename R>
 void launch_efield(const R* phi, int gx, int gy, int gz, const DomainRec* dom,
                    typename vec4<R>::type* E, hipStream_t st);

@@ -1958,7 +1958,7 @@ void launch_reorder_records(double* parts, int64_t stride, uint8_t* masks, int64
 template <bool UNIT>
 static void launch_deposit_tiles(const double* parts, int64_t stride, const uint8_t* masks,
                                  const int32_t* perm, int64_t n, int gx, int gy, int gz,
-                                 DomainRec* dom, double* rho, hipStream_t st)
+                                 DomainRec* dom, double* rho, bool served, hipStream_t st)
 {
     auto launch = [&](auto kernel, int per) {
         const int64_t win = kTileThreads * int64_t(per), nb = (n + win - 1) / win;
@@ -1971,36 +1971,34 @@ static void launch_deposit_tiles(const double* parts, int64_t stride, const uint
     // / 11.6 on 32x32x64; 4e5 on 64x64x128 14.8 / 12.6 / 15.5; 1e6 23.4 / 20.6 /
     // 19.9); one through a permutation, whose random reads want the wavefronts
     // (1e5 11.1 / 12.4 / 18.0, 1e6 25.2 / 25.8 / 31.6, 4e6 82.8 / 81.8 / 84.1).
-    // The precision form keeps four everywhere: its windows are the groups that
-    // are rounded together, and smaller ones move a sparse bunch's field by
-    // more than its earlier results differ among themselves (n < 60000: dp/p by
-    // 1e-8 where they differ by 2e-9).
-    if (perm != nullptr) {
+    // The precision form's windows are the groups that are rounded together, and
+    // smaller ones move a sparse bunch's field by more than the results of four
+    // slots ever differed among themselves (n < 60000: dp/p by 1e-8 where they
+    // differ by 2e-9), so an operator's applies keep four.  A server's, whose
+    // jobs' results are emittances and moments (1e-9), take the same rule as
+    // FP64 (128 mixed jobs: 3.29 -> 3.22 s).
+    if (perm != nullptr)
         launch(k_deposit_tile<UNIT, 1, true>, 1);
-        return;
-    }
-    if constexpr (!UNIT) {
-        if (n < 250000) {
-            launch(k_deposit_tile<UNIT, 1, false>, 1);
-            return;
-        }
-        if (n < 750000) {
-            launch(k_deposit_tile<UNIT, 2, false>, 2);
-            return;
-        }
-    }
-    launch(k_deposit_tile<UNIT, 4, false>, 4);
+    else if (UNIT && !served)
+        launch(k_deposit_tile<UNIT, 4, false>, 4);
+    else if (n < 250000)
+        launch(k_deposit_tile<UNIT, 1, false>, 1);
+    else if (n < 750000)
+        launch(k_deposit_tile<UNIT, 2, false>, 2);
+    else
+        launch(k_deposit_tile<UNIT, 4, false>, 4);
 }
 
 void launch_deposit(const double* parts, int64_t stride, const uint8_t* masks,
                     const int32_t* perm, int64_t n, int gx, int gy, int gz, DomainRec* dom,
-                    double* sums, float* rho32, hipStream_t st)
+                    double* sums, float* rho32, bool served, hipStream_t st)
 {
     if (!rho32) {
-        launch_deposit_tiles<false>(parts, stride, masks, perm, n, gx, gy, gz, dom, sums, st);
+        launch_deposit_tiles<false>(parts, stride, masks, perm, n, gx, gy, gz, dom, sums, served,
+                                    st);
         return;
     }
-    launch_deposit_tiles<true>(parts, stride, masks, perm, n, gx, gy, gz, dom, sums, st);
+    launch_deposit_tiles<true>(parts, stride, masks, perm, n, gx, gy, gz, dom, sums, served, st);
     const int64_t G = int64_t(gx) * gy * gz;
     hipLaunchKernelGGL(k_rho_round, dim3(grid_for(G / 16, 256)), dim3(kThreads), 0, st, sums, rho32,
                        G, dom);
