@@ -321,7 +321,9 @@ __device__ __forceinline__ void fast_slice_apply(FastDrift& f, const PreparedSli
 // The whole program on one particle: the fast form; in a wavefront with a
 // particle out of its range (tested after every slice) the rolled form from the
 // start state, which `again` brings back (re-read rather than held: 10
-// registers over the fast loop); the general form for what is left.
+// registers over the fast loop); the general form for what is left.  4e6
+// particles, O-F-O-D, one at |x'| = 0.8 per wavefront: 742 us (515 without; the
+// whole fast program and then the general one 1063).
 template <typename Again>
 __device__ __forceinline__ void apply_program(const MapProgram& prog, double& x, double& xp,
                                               double& y, double& yp, double& cdt, double dpop,
