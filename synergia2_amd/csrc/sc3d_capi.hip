@@ -518,7 +518,11 @@ int sc3d_apply(sc3d_ctx* c, const sc3d_bunch* b, double time_step, void* stream)
     // the cross-stream fork and join cost more than the overlap gives
     // (measured at 1e5 particles on 32x32x64, synchronised every step: 0.095
     // -> 0.150 ms per step with the fork; on the 64-job mix 2.08e9 -> 2.03e9
-    // particle-steps/s when every apply of a grid of 2^18 cells forked).
+    // particle-steps/s when every apply of a grid of 2^18 cells forked).  The
+    // line was drawn with a longer deposit and sort; with the present ones the
+    // overlap gives less (tracking ahead with the maps fused, us per step
+    // without / with the fork: 64x64x128 FP64 1e6 150 / 163, 2e6 206 / 216, 4e6
+    // 309 / 316, FP32 4e6 297 / 298; 128x128x256 FP32 1.6e7 1250 / 1240).
     const bool eligible = c->timing != SC3D_TIMING_PHASES &&
                           int64_t(c->g.gx) * c->g.gy * c->g.gz >= (int64_t(1) << 18) &&
                           b->n_active >= (int64_t(1) << 20);
